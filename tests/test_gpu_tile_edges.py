@@ -1,0 +1,80 @@
+"""Kernels at the sizes where their tiles, chunks and dispatch rules end,
+against the CPU oracle (bit for bit) or an FP64 reference."""
+import numpy as np
+import pytest
+import torch
+
+import damascene_amd as dm
+from damascene_amd import autograd as AG
+from oracle import grad_ref as G
+from oracle import pyoracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def host(t):
+    return t.cpu().numpy()
+
+
+def bits(a):
+    return np.ascontiguousarray(a).view(np.uint32)
+
+
+# spectral Pb: 64 x 4 pixel blocks, eight vectors staged at a time, taken in pairs
+@pytest.mark.parametrize("w,h,nvec", [(32, 32, 2), (64, 36, 9), (65, 37, 10), (129, 33, 17), (33, 41, 32)])
+def test_spectral_pb_tiles(ctx, w, h, nvec):
+    print(f"case: spectral Pb {w}x{h}, {nvec} vectors", flush=True)
+    r = np.random.RandomState(w + nvec)
+    vecs = r.rand(nvec, h, w).astype(np.float32)
+    vals = np.sort(r.rand(nvec)).astype(np.float32) + 1e-4
+    got = host(ctx.spectral_pb(vals, ctx.upload(vecs)))[:, :w * h]
+    assert np.array_equal(bits(got), bits(O.spectral_pb(vals, vecs, w, h).reshape(8, -1)))
+
+
+# the differentiable pair: the same blocks forward, 32 x 8 pixel blocks and
+# eight vectors a chunk in the eigenvector gradient
+@pytest.mark.parametrize("w,h,nvec", [(32, 32, 2), (65, 37, 9), (64, 40, 10), (97, 33, 16)])
+def test_spb_combine_tiles(ctx, w, h, nvec):
+    print(f"case: spectral Pb + combine gradients {w}x{h}, {nvec} vectors", flush=True)
+    r = np.random.RandomState(7 * w + nvec)
+    n = w * h
+    cues = [r.rand(24, n).astype(np.float32) for _ in range(4)]
+    vecs = r.rand(nvec, h, w).astype(np.float32)
+    params = np.concatenate([r.rand(12) * 0.02, [0.0139], r.rand(nvec) * 3 + 1]).astype(np.float32)
+    grad = r.randn(h, w).astype(np.float32)
+    op = AG.SpbCombine(ctx, w, h, [ctx.upload(c) for c in cues])
+    p = ctx.upload(params).requires_grad_(True)
+    v = ctx.upload(vecs).requires_grad_(True)
+    pre = op(p, v)
+    pre.backward(ctx.upload(grad))
+    C = G.cue_planes(*cues, w, h)
+    p64 = torch.as_tensor(params, dtype=torch.float64).requires_grad_(True)
+    v64 = torch.as_tensor(vecs, dtype=torch.float64).requires_grad_(True)
+    all64, R64 = G.parts64(p64, v64, C, w, h)
+    (all64.max(0).values * torch.as_tensor(grad, dtype=torch.float64)).sum().backward()
+    # FP32: a response is a chain of 49 fused multiply-adds of values below 1
+    # with weights of unit L1 norm (error below 49 * 2^-24 = 2.9e-6), a plane
+    # sums 12 + nvec of them
+    top = all64.detach().max(0).values
+    assert float((pre.detach().cpu().double() - top).abs().max()) < 1e-5 * float(all64.detach().abs().max())
+    # the gradients agree where FP32 cannot route them elsewhere: no near-tie
+    # of the maximising orientation or of a response's sign in the pixel's
+    # 7 x 7 window (bounds as in test_backward_against_fp64)
+    gv, gv64 = host(v.grad), v64.grad.numpy()
+    s = np.sort(all64.detach().numpy(), axis=0)[-2:]
+    tie = s[1] - s[0] < 1e-5 * s.max()
+    ostar = all64.detach().numpy().argmax(axis=0)
+    rstar = np.take_along_axis(np.abs(R64.detach().numpy()), ostar[None, None], axis=1)[:, 0]
+    for i in range(1, nvec):
+        amb = tie | (rstar[i - 1] < 1e-5)
+        near = np.zeros_like(amb)
+        for dy in range(-3, 4):
+            for dx in range(-3, 4):
+                near |= np.roll(np.roll(amb, dy, 0), dx, 1)
+        assert np.abs(gv[i] - gv64[i])[~near].max() < 1e-4 * np.abs(gv64).max(), f"vector {i}"
+    assert np.all(gv[0] == 0)
+    # parameters: FP64 block sums of FP32 terms; an ambiguous pixel may move
+    # its own term
+    gp, gp64 = host(p.grad), p64.grad.numpy()
+    assert np.abs(gp - gp64).max() < (1e-5 + 2.0 * tie.sum() / n) * np.abs(gp64).max()
+    assert gp[13] == 0
