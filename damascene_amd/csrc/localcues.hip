@@ -41,7 +41,8 @@ struct FrameGeom {
   int nw[4], nh[4];
   long long lab_off[kFrames];  // byte offset of frame f = ch*4 + o (label buffer)
   long long int_off[kFrames];  // uint16 element offset of frame f (integral buffer)
-  long long band_off[kFrames];  // uint16 element offset of frame f's band sums (k_integral_band)
+  long long band_off[kFrames];  // uint16 element offset of frame f's band sums (k_integral_strip)
+  long long row_off[kFrames];   // uint32 word offset of frame f's row carries (k_integral_strip)
   int tab_off[4];              // offset of orientation o's tables: bX[bw] bY[bw] gX[bh] gY[bh]
   int rect[4][4][8];           // [orientation][radius index][corner A..H]
   int tbp;                     // bins per integral pixel of the texture frames (32 or 64)
@@ -151,141 +152,211 @@ __global__ __launch_bounds__(256) void k_integral_cols(FrameGeom g, int f0, uint
   }
 }
 
-// Single-write integral images.  A frame is cut into bands of kBand rows;
-// I(x, y) for y in band b is the carry C_b(x) = sum over earlier bands of
-// their row-prefixed column counts P_b'(x) plus the band's own running sum of
-// row prefixes.  Pass 1 (FINAL = false) leaves P_b per band, k_band_carry
-// turns them into the exclusive prefix over bands in place, pass 2 (FINAL)
-// starts each band's running sums at its carry and writes every integral
-// value once.  One block of 1024 threads per (band, frame); thread t owns
-// columns x = t + 1024 c (c < NCH) and keeps their running sums for all
-// bins in registers (two u16 bins per word, modulo 2^16 like the stored
-// integrals).  The row prefix of bin k at column x is the count of k among
-// the lanes below x in its wave (ballot + mbcnt) plus the exclusive total
-// of the earlier waves (their totals through LDS, one barrier per row).
-// Each thread stores its pixel's BP bins as BP/8 16-byte plane entries, so
-// a wave's store to one plane is one contiguous kilobyte.
+// Single-write integral images.  A frame is cut into bands of kBand rows and
+// strips of 64 columns; one wave owns a (strip, band) and lane x one column.
+// Going down the band's rows it keeps, per bin, the running sum of the
+// strip's row prefixes, L(x, y) = number of the bin's labels in the strip's
+// columns <= x of the band's rows <= y: per row and bin a compare, the two
+// mbcnt instructions that count the wave's matching lanes below (accumulating
+// into L) and an add with carry for the lane's own match.  Then
+//   I(x, y) = C_b(x) + R_s(y) + L(x, y)  (modulo 2^16 per bin)
+// with R_s(y) the same sum over the band's strips left of s (the last lane's
+// L of those strips, scanned over the strips by k_strip_carry) and C_b(x)
+// that of the earlier bands' last rows (k_band_carry).  Pass 1 (FINAL =
+// false) leaves each row's last-lane L and each band's last row; pass 2
+// recomputes L and writes every integral value once: a wave's store to one
+// plane is one contiguous kilobyte.  No barriers and no LDS: with one block
+// per band whose 16 waves exchanged their row totals through LDS at a
+// barrier per row the two passes took 143 + 126 us (L/a/b frames) and 55 +
+// 51 us (texton frames) at 481x321, and take 64 + 30 and 30 + 17 us.  Pass 1
+// is bound by its VALU instructions (about 8 per pixel and bin pair).
 constexpr int kBand = 16;
-constexpr int kIntThreads = 1024, kIntWaves = kIntThreads / 64;
+constexpr int kStrip = 64;
 
-template <int BP, int NBU, int NCH, bool FINAL>
-__global__ __launch_bounds__(kIntThreads) void k_integral_band(FrameGeom g, int f0,
-                                                               const uint8_t* __restrict__ frames,
-                                                               uint16_t* __restrict__ bands,
-                                                               uint16_t* __restrict__ I) {
-  constexpr int NQ = BP / 2;  // words per record (two bins each)
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t add_u16x2(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, a) + __builtin_bit_cast(u16x2, b));
+}
+
+template <int BP, int NBU, bool FINAL>
+__global__ __launch_bounds__(256) void k_integral_strip(FrameGeom g, int f0, int4 first,
+                                                        const uint8_t* __restrict__ frames,
+                                                        uint16_t* __restrict__ bands, uint32_t* __restrict__ rows,
+                                                        const uint32_t* __restrict__ carry,
+                                                        uint16_t* __restrict__ I) {
+  constexpr int NQ = BP / 2;          // words per record (two bins each)
   constexpr int NQU = (NBU + 1) / 2;  // words holding used bins (labels are < NBU; higher bins stay 0)
-  constexpr int NS = NCH * kIntWaves;
-  __shared__ uint32_t tot[2][NS][NBU];  // per-wave bin totals, by row parity
-  const int f = f0 + blockIdx.y, o = f & 3, b = blockIdx.x;
-  const int nw = g.nw[o], nh = g.nh[o];
+  // blocks of a channel's four frames follow each other: first = the first
+  // block of orientations 1, 2, 3 and of the next channel; numbered
+  // XCD-aware, so neighbouring strips, whose stores share cache lines (a
+  // frame's rows are not line-aligned), mostly meet in one L2
+  const int lb = dev::xcd_block(blockIdx.x, gridDim.x);
+  const int ch = lb / first.w, in_ch = lb - ch * first.w;
+  const int o = in_ch < first.x ? 0 : in_ch < first.y ? 1 : in_ch < first.z ? 2 : 3, f = f0 + 4 * ch + o;
+  const int blk = in_ch - (o == 0 ? 0 : o == 1 ? first.x : o == 2 ? first.y : first.z);
+  const int nw = g.nw[o], nh = g.nh[o], ns = (nw + kStrip - 1) / kStrip;
+  const int lane = threadIdx.x & 63;
+  const int unit = blk * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int b = unit / ns, s = unit - b * ns;
   const int y0 = b * kBand;
-  if (y0 >= nh) return;  // the whole block: past this frame's last band
-  const int y1 = min(nh, y0 + kBand);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  uint16_t* bsum = bands + g.band_off[f] + (size_t)b * nw * BP;
-  uint32_t S[NCH][NQ];
+  if (y0 >= nh) return;  // past this frame's last band
+  const int y1 = min(nh, y0 + kBand), x = s * kStrip + lane;
+  const bool in = x < nw;
+  uint32_t L[2 * NQU];
 #pragma unroll
-  for (int c = 0; c < NCH; c++) {
-    const int x = c * kIntThreads + (int)threadIdx.x;
+  for (int k = 0; k < 2 * NQU; k++) L[k] = 0;
+  uint16_t* rec = bands + g.band_off[f] + ((size_t)b * nw + (in ? x : 0)) * BP;
+  uint32_t C[NQU];
 #pragma unroll
-    for (int q = 0; q < NQ; q += 4) {
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (FINAL && x < nw) v = *reinterpret_cast<const uint4*>(bsum + (size_t)x * BP + 2 * q);
-      S[c][q] = v.x;
-      S[c][q + 1] = v.y;
-      S[c][q + 2] = v.z;
-      S[c][q + 3] = v.w;
-    }
+  for (int q = 0; q < NQU; q++) C[q] = 0;
+  if (FINAL) {
+#pragma unroll
+    for (int q = 0; q < NQ; q += 4)
+      if (q < NQU) {
+        const uint4 v = *reinterpret_cast<const uint4*>(rec + 2 * q);
+        C[q] = v.x;
+        if (q + 1 < NQU) C[q + 1] = v.y;
+        if (q + 2 < NQU) C[q + 2] = v.z;
+        if (q + 3 < NQU) C[q + 3] = v.w;
+      }
   }
-  const uint8_t* lab_base = frames + g.lab_off[f];
-  uint32_t labn[NCH];  // the next row's labels, loaded one row ahead
+  const uint8_t* lab = frames + g.lab_off[f] + x;
+  size_t row = (size_t)g.row_off[f] + ((size_t)y0 * ns + s) * NQ;  // this row's and strip's record
+  const size_t npx = (size_t)nw * nh;
+  uint4* dst = reinterpret_cast<uint4*>(I + g.int_off[f]) + (size_t)y0 * nw + x;
+  constexpr int kAhead = 4;  // rows whose labels are loaded together, one group ahead
+  uint32_t next[kAhead];
 #pragma unroll
-  for (int c = 0; c < NCH; c++) {
-    const int x = c * kIntThreads + (int)threadIdx.x;
-    labn[c] = x < nw ? (uint32_t)lab_base[(size_t)y0 * nw + x] : 255u;
-  }
-  for (int y = y0; y < y1; y++) {
-    const int par = (y - y0) & 1;
-    uint32_t lab[NCH];
+  for (int r = 0; r < kAhead; r++) next[r] = in && y0 + r < y1 ? (uint32_t)lab[(size_t)(y0 + r) * nw] : 255u;
+#pragma unroll 1
+  for (int yb = y0; yb < y1; yb += kAhead) {
+    uint32_t cur[kAhead];
 #pragma unroll
-    for (int c = 0; c < NCH; c++) {
-      lab[c] = labn[c];
-      const int x = c * kIntThreads + (int)threadIdx.x;
-      labn[c] = (y + 1 < y1 && x < nw) ? (uint32_t)lab_base[(size_t)(y + 1) * nw + x] : 255u;
+    for (int r = 0; r < kAhead; r++) {
+      cur[r] = next[r];
+      const int y = yb + kAhead + r;
+      next[r] = in && y < y1 ? (uint32_t)lab[(size_t)y * nw] : 255u;
     }
-    uint32_t Rl[NCH][NQU];
 #pragma unroll
-    for (int c = 0; c < NCH; c++) {
+    for (int r = 0; r < kAhead; r++) {
+      if (yb + r >= y1) break;
+      uint32_t R[NQU];
 #pragma unroll
-      for (int q = 0; q < NQU; q++) {
-        const unsigned long long m0 = __ballot(lab[c] == (uint32_t)(2 * q));
-        const uint32_t r0 = __builtin_amdgcn_mbcnt_hi((uint32_t)(m0 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m0, 0u)) +
-                            (lab[c] == (uint32_t)(2 * q));
-        uint32_t r1 = 0;
-        if (2 * q + 1 < NBU) {
-          const unsigned long long m1 = __ballot(lab[c] == (uint32_t)(2 * q + 1));
-          r1 = __builtin_amdgcn_mbcnt_hi((uint32_t)(m1 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m1, 0u)) +
-               (lab[c] == (uint32_t)(2 * q + 1));
-          if (lane == 0) tot[par][c * kIntWaves + wv][2 * q + 1] = (uint32_t)__popcll(m1);
+      for (int q = 0; q < NQU; q++) R[q] = FINAL ? carry[row + q] : 0u;  // wave-uniform: scalar loads
+#pragma unroll
+      for (int k0 = 0; k0 < NBU; k0 += 5) {  // five masks at a time: none is read right after its compare
+        unsigned long long m[5];
+#pragma unroll
+        for (int k = k0; k < k0 + 5 && k < NBU; k++) m[k - k0] = __ballot(cur[r] == (uint32_t)k);
+#pragma unroll
+        for (int k = k0; k < k0 + 5 && k < NBU; k++)
+          L[k] = __builtin_amdgcn_mbcnt_hi((uint32_t)(m[k - k0] >> 32),
+                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m[k - k0], L[k])) +
+                 (cur[r] == (uint32_t)k);
+      }
+      uint32_t W[NQ];
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        W[q] = 0;
+        if (q < NQU) {
+          W[q] = __builtin_amdgcn_perm(L[2 * q + 1], L[2 * q], 0x05040100u);  // low halves
+          if (FINAL) W[q] = add_u16x2(add_u16x2(W[q], C[q]), R[q]);
         }
-        if (lane == 0) tot[par][c * kIntWaves + wv][2 * q] = (uint32_t)__popcll(m0);
-        Rl[c][q] = r0 | (r1 << 16);
       }
-    }
-    __syncthreads();
+      if (FINAL) {
+        if (in)
 #pragma unroll
-    for (int c = 0; c < NCH; c++) {
-      const int x = c * kIntThreads + (int)threadIdx.x;
-      // bin `lane`'s count over the row's earlier waves, then broadcast per bin
-      uint32_t pv = 0;
-      if (lane < NBU)
-        for (int k = 0; k < c * kIntWaves + wv; k++) pv += tot[par][k][lane];
+          for (int q = 0; q < NQ; q += 4) dst[(size_t)(q / 4) * npx] = make_uint4(W[q], W[q + 1], W[q + 2], W[q + 3]);
+      } else {
+        uint4* rd = reinterpret_cast<uint4*>(rows + row);
+        if (lane == kStrip - 1)
 #pragma unroll
-      for (int q = 0; q < NQU; q++) {
-        // row prefix of bins 2q, 2q+1 (each below 2^16: no carry between halves)
-        const uint32_t p0 = (uint32_t)__builtin_amdgcn_readlane((int)pv, 2 * q);
-        const uint32_t p1 = 2 * q + 1 < NBU ? (uint32_t)__builtin_amdgcn_readlane((int)pv, 2 * q + 1) : 0u;
-        const uint32_t r = Rl[c][q] + (p0 | (p1 << 16));
-        const uint32_t lo = (S[c][q] + r) & 0xffffu;
-        const uint32_t hi = ((S[c][q] >> 16) + (r >> 16)) << 16;
-        S[c][q] = lo | hi;
+          for (int q = 0; q < NQ; q += 4) rd[q / 4] = make_uint4(W[q], W[q + 1], W[q + 2], W[q + 3]);
+        if (in && yb + r == y1 - 1) {
+          uint4* bd = reinterpret_cast<uint4*>(rec);
+#pragma unroll
+          for (int q = 0; q < NQ; q += 4) bd[q / 4] = make_uint4(W[q], W[q + 1], W[q + 2], W[q + 3]);
+        }
       }
-      if (FINAL && x < nw) {
-        // plane q / 4 of this pixel: 16 bytes; consecutive lanes, consecutive pixels
-        const size_t npx = (size_t)nw * nh;
-        uint4* dst = reinterpret_cast<uint4*>(I + g.int_off[f]) + (size_t)y * nw + x;
-#pragma unroll
-        for (int q = 0; q < NQ; q += 4) dst[(q / 4) * npx] = make_uint4(S[c][q], S[c][q + 1], S[c][q + 2], S[c][q + 3]);
-      }
-    }
-  }
-  if (!FINAL) {
-#pragma unroll
-    for (int c = 0; c < NCH; c++) {
-      const int x = c * kIntThreads + (int)threadIdx.x;
-      if (x < nw) {
-        uint4* dst = reinterpret_cast<uint4*>(bsum + (size_t)x * BP);
-#pragma unroll
-        for (int q = 0; q < NQ; q += 4) dst[q / 4] = make_uint4(S[c][q], S[c][q + 1], S[c][q + 2], S[c][q + 3]);
-      }
+      row += (size_t)ns * NQ;
+      dst += nw;
     }
   }
 }
 
-// Band sums -> exclusive prefix over the bands of each frame (in place).
-__global__ __launch_bounds__(256) void k_band_carry(FrameGeom g, int f0, uint16_t* __restrict__ bands) {
+// Rows of last-lane sums -> exclusive prefix over the row's strips (in
+// place); one thread per (row, word).
+__global__ __launch_bounds__(256) void k_strip_carry(FrameGeom g, int f0, uint32_t* __restrict__ rows) {
   const int f = f0 + blockIdx.y, o = f & 3;
-  const int nw = g.nw[o], nb = (g.nh[o] + kBand - 1) / kBand, bp = bin_pitch(g, f);
+  const int ns = (g.nw[o] + kStrip - 1) / kStrip, nq = bin_pitch(g, f) / 2;
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nw * bp) return;
-  uint16_t* p = bands + g.band_off[f] + e;
-  const size_t stride = (size_t)nw * bp;
-  uint16_t acc = 0;
-  for (int b = 0; b < nb; b++) {
-    const uint16_t t = p[(size_t)b * stride];
-    p[(size_t)b * stride] = acc;
-    acc = (uint16_t)(acc + t);
+  if (e >= g.nh[o] * nq) return;
+  const int y = e / nq, q = e - y * nq;
+  uint32_t* p = rows + g.row_off[f] + (size_t)y * ns * nq + q;
+  uint32_t acc = 0;
+  for (int s0 = 0; s0 < ns; s0 += 8) {
+    uint32_t t[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) t[k] = s0 + k < ns ? p[(size_t)(s0 + k) * nq] : 0u;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      if (s0 + k < ns) p[(size_t)(s0 + k) * nq] = acc;
+      acc = add_u16x2(acc, t[k]);
+    }
+  }
+}
+
+// Each band's last row, completed by its strips' carries, -> exclusive
+// prefix over the bands of each frame (in place).  A block owns 32 pieces of
+// a row (one column's 16 bytes each) and 8 groups of threads that share the
+// frame's bands: every group sums its bands, the groups' sums meet in LDS,
+// and each writes its bands' prefixes (one chain over 58 bands per thread
+// was 20 us at 481x321 for the L/a/b and for the texton frames; this is 11).
+constexpr int kCarryCols = 32, kCarrySegs = 8;
+__global__ __launch_bounds__(256) void k_band_carry(FrameGeom g, int f0, const uint32_t* __restrict__ rows,
+                                                    uint16_t* __restrict__ bands) {
+  __shared__ uint4 sums[kCarrySegs][kCarryCols];
+  const int f = f0 + blockIdx.y, o = f & 3;
+  const int nw = g.nw[o], nh = g.nh[o], nb = (nh + kBand - 1) / kBand, n4 = bin_pitch(g, f) / 8;
+  const int ns = (nw + kStrip - 1) / kStrip;
+  const int c = threadIdx.x % kCarryCols, seg = threadIdx.x / kCarryCols;
+  const int e = blockIdx.x * kCarryCols + c;
+  const bool in = e < nw * n4;
+  const int s = in ? e / n4 / kStrip : 0, q = in ? e % n4 : 0;
+  uint4* p = reinterpret_cast<uint4*>(bands + g.band_off[f]) + (in ? e : 0);
+  const uint4* r = reinterpret_cast<const uint4*>(rows + g.row_off[f]) + (size_t)s * n4 + q;
+  const size_t stride = (size_t)nw * n4;
+  const int per = (nb + kCarrySegs - 1) / kCarrySegs, b0 = seg * per, b1 = min(nb, b0 + per);
+  auto add = [](uint4& a, const uint4& v) {
+    a.x = add_u16x2(a.x, v.x);
+    a.y = add_u16x2(a.y, v.y);
+    a.z = add_u16x2(a.z, v.z);
+    a.w = add_u16x2(a.w, v.w);
+  };
+  auto band = [&](int b) {
+    uint4 t = p[(size_t)b * stride];
+    add(t, r[(size_t)(min(nh, (b + 1) * kBand) - 1) * ns * n4]);
+    return t;
+  };
+  uint4 acc = make_uint4(0u, 0u, 0u, 0u);
+  if (in)
+#pragma unroll 8
+    for (int b = b0; b < b1; b++) add(acc, band(b));
+  sums[seg][c] = acc;
+  __syncthreads();
+  acc = make_uint4(0u, 0u, 0u, 0u);
+  for (int k = 0; k < seg; k++) add(acc, sums[k][c]);
+  if (!in) return;
+  for (int b = b0; b < b1; b += 4) {
+    uint4 t[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) t[k] = band(min(b + k, nb - 1));
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (b + k < b1) {
+        p[(size_t)(b + k) * stride] = acc;
+        add(acc, t[k]);
+      }
   }
 }
 
@@ -313,7 +384,6 @@ __device__ __forceinline__ float chi2_split(const uint32_t (&pk)[8][16], int i0,
   float a[32], b[32];
   // two bins per 32-bit word: the corner sums in packed 16-bit arithmetic,
   // each half modulo 2^16 on its own
-  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
   for (int e = 0; e < 16; e++) {
     if (2 * e < NB) {
@@ -567,8 +637,7 @@ size_t parabola_lds() {
 struct CuePlan {
   int w = -1, h = -1;
   FrameGeom g;
-  size_t lab_bytes = 0, int_elems = 0, band_elems = 0;
-  bool band_ok = false;  // frames narrow enough for the single-write integral pass
+  size_t lab_bytes = 0, int_elems = 0, band_elems = 0, row_words = 0;
   int tap_stride = 0;
   int* d_tabs = nullptr;
   float* d_coef[4] = {nullptr, nullptr, nullptr, nullptr};  // [8][2r+1][2r+1] per radius
@@ -631,26 +700,22 @@ int build_plan(hipStream_t s, int w, int h, int tbp, CuePlan& P) {
           return fail(DMSC_ERR_INTERNAL, "half-disc corners leave the frame (o=%d)", o);
       }
   }
-  size_t lo = 0, io = 0, bo = 0;
+  size_t lo = 0, io = 0, bo = 0, ro = 0;
   for (int f = 0; f < kFrames; f++) {
     const int o = f & 3;
     g.lab_off[f] = (long long)lo;
     g.int_off[f] = (long long)io;
     g.band_off[f] = (long long)bo;
+    g.row_off[f] = (long long)ro;
     lo += ((size_t)g.nw[o] * g.nh[o] + 255) & ~(size_t)255;
     io += (size_t)g.nw[o] * g.nh[o] * (f >= 12 ? tbp : 32);
     bo += (size_t)div_up(g.nh[o], kBand) * g.nw[o] * (f >= 12 ? tbp : 32);
+    ro += (size_t)g.nh[o] * div_up(g.nw[o], kStrip) * (f >= 12 ? tbp : 32) / 2;
   }
   P.lab_bytes = lo;
   P.int_elems = io;
   P.band_elems = bo;
-  // the single-write integral pass covers frames up to 2 * kIntThreads
-  // columns; wider ones use the row + column passes
-  {
-    int maxw = 0;
-    for (int o = 0; o < 4; o++) maxw = std::max(maxw, g.nw[o]);
-    P.band_ok = maxw <= 2 * kIntThreads;
-  }
+  P.row_words = ro;
   DMSC_HIP(hipMalloc(&P.d_tabs, sizeof(int) * tabs.size()));
   DMSC_HIP(hipMemcpy(P.d_tabs, tabs.data(), sizeof(int) * tabs.size(), hipMemcpyHostToDevice));
   for (int ri = 0; ri < 4; ri++) {
@@ -685,27 +750,43 @@ int build_plan(hipStream_t s, int w, int h, int tbp, CuePlan& P) {
   return DMSC_OK;
 }
 
-// Integral images of frames f0 .. f0 + nf - 1 (BP bins) in three launches:
-// band sums, carries, final pass (frames up to 2 * kIntThreads wide).
-template <int BP, int NBU, int NCH>
-int integral_bands_n(hipStream_t s, const FrameGeom& g, int f0, int nf, int maxw, int maxh, const uint8_t* frames,
-                     uint16_t* bands, uint16_t* I) {
-  const dim3 grid(div_up(maxh, kBand), nf);
-  hipLaunchKernelGGL((k_integral_band<BP, NBU, NCH, false>), grid, dim3(kIntThreads), 0, s, g, f0, frames, bands,
-                     I);
-  hipLaunchKernelGGL(k_band_carry, dim3(div_up(maxw * BP, 256), nf), dim3(256), 0, s, g, f0, bands);
-  hipLaunchKernelGGL((k_integral_band<BP, NBU, NCH, true>), grid, dim3(kIntThreads), 0, s, g, f0, frames, bands, I);
+// Integral images of frames f0 .. f0 + nf - 1: BP bins per record, NBU of
+// them used (the L/a/b frames hold 25 quantised bins in 32-bin records; the
+// unused bins stay 0).
+template <int BP, int NBU>
+int integral_strips(hipStream_t s, const FrameGeom& g, int f0, int nf, const uint8_t* frames, uint16_t* bands,
+                    uint32_t* rows, uint16_t* I) {
+  int first[5] = {0}, row_words = 0, col_quads = 0;
+  for (int o = 0; o < 4; o++) {
+    first[o + 1] = first[o] + div_up(div_up(g.nw[o], kStrip) * div_up(g.nh[o], kBand), 4);
+    row_words = std::max(row_words, g.nh[o] * (BP / 2));
+    col_quads = std::max(col_quads, g.nw[o] * (BP / 8));
+  }
+  const int4 at = make_int4(first[1], first[2], first[3], first[4]);
+  const dim3 grid(first[4] * (nf / 4));
+  hipLaunchKernelGGL((k_integral_strip<BP, NBU, false>), grid, dim3(256), 0, s, g, f0, at, frames, bands,
+                     rows, nullptr, nullptr);
+  hipLaunchKernelGGL(k_strip_carry, dim3(div_up(row_words, 256), nf), dim3(256), 0, s, g, f0, rows);
+  hipLaunchKernelGGL(k_band_carry, dim3(div_up(col_quads, kCarryCols), nf), dim3(256), 0, s, g, f0, rows, bands);
+  hipLaunchKernelGGL((k_integral_strip<BP, NBU, true>), grid, dim3(256), 0, s, g, f0, at, frames, bands,
+                     nullptr, rows, I);
   DMSC_HIP(hipGetLastError());
   return DMSC_OK;
 }
 
-// BP bins per record, NBU of them used (the L/a/b frames hold 25 quantised
-// bins in 32-bin records; the unused bins stay 0)
-template <int BP, int NBU>
-int integral_bands(hipStream_t s, const FrameGeom& g, int f0, int nf, int maxw, int maxh, const uint8_t* frames,
-                   uint16_t* bands, uint16_t* I) {
-  if (maxw <= kIntThreads) return integral_bands_n<BP, NBU, 1>(s, g, f0, nf, maxw, maxh, frames, bands, I);
-  return integral_bands_n<BP, NBU, 2>(s, g, f0, nf, maxw, maxh, frames, bands, I);
+// Byte offsets in the scratch arena: label frames (at 0), integral images,
+// raw gradient planes, band sums, row carries.
+struct ScratchLayout {
+  size_t ints, grads, bands, rows, total;
+};
+ScratchLayout scratch_layout(const CuePlan& P) {
+  ScratchLayout a;
+  a.ints = P.lab_bytes;
+  a.grads = a.ints + P.int_elems * sizeof(uint16_t);
+  a.bands = a.grads + (size_t)4 * 24 * P.w * P.h * sizeof(float);
+  a.rows = a.bands + P.band_elems * sizeof(uint16_t);
+  a.total = a.rows + P.row_words * sizeof(uint32_t) + 1024;
+  return a;
 }
 
 struct PlanCache {
@@ -773,9 +854,7 @@ int local_cues_prepare(Ctx* ctx, int w, int h, int ntex) {
   CuePlan* P;
   DMSC_TRY(get_plan(ctx, w, h, ntex, &P));
   void* scratch;
-  const size_t gbytes = (size_t)4 * 24 * w * h * sizeof(float);
-  return ctx->scratch(1, P->lab_bytes + P->int_elems * sizeof(uint16_t) + gbytes + P->band_elems * sizeof(uint16_t) + 1024,
-                      &scratch);
+  return ctx->scratch(1, scratch_layout(*P).total, &scratch);
 }
 
 int launch_local_cues_part(Ctx* ctx, hipStream_t s, int part, int w, int h, const float* L, const float* A,
@@ -789,13 +868,13 @@ int launch_local_cues_part(Ctx* ctx, hipStream_t s, int part, int w, int h, cons
   const FrameGeom& g = P->g;
   const int n = w * h;
   void* scratch;
-  const size_t gbytes = (size_t)4 * 24 * n * sizeof(float);
-  const size_t ibytes = P->int_elems * sizeof(uint16_t);
-  DMSC_TRY(ctx->scratch(1, P->lab_bytes + ibytes + gbytes + P->band_elems * sizeof(uint16_t) + 1024, &scratch));
+  const ScratchLayout at = scratch_layout(*P);
+  DMSC_TRY(ctx->scratch(1, at.total, &scratch));
   uint8_t* frames = (uint8_t*)scratch;
-  uint16_t* I = (uint16_t*)((char*)scratch + P->lab_bytes);
-  float* grads = grads_out ? grads_out : (float*)((char*)scratch + P->lab_bytes + ibytes);
-  uint16_t* bands = (uint16_t*)((char*)scratch + P->lab_bytes + ibytes + gbytes);
+  uint16_t* I = (uint16_t*)((char*)scratch + at.ints);
+  float* grads = grads_out ? grads_out : (float*)((char*)scratch + at.grads);
+  uint16_t* bands = (uint16_t*)((char*)scratch + at.bands);
+  uint32_t* rows = (uint32_t*)((char*)scratch + at.rows);
   const bool colour = part & 1, texture = part & 2;
   // frames of channel ch are f = 4 ch + o; the texture frames 12..15 come last
   const size_t split = (size_t)g.lab_off[12];
@@ -807,17 +886,17 @@ int launch_local_cues_part(Ctx* ctx, hipStream_t s, int part, int w, int h, cons
   int maxh = 0, maxw = 0;
   for (int o = 0; o < 4; o++) { maxh = std::max(maxh, g.nh[o]); maxw = std::max(maxw, g.nw[o]); }
   if (colour) {
-    if (P->band_ok && integral_pass == 1) {
-      DMSC_TRY((integral_bands<32, 25>(s, g, 0, 12, maxw, maxh, frames, bands, I)));
+    if (integral_pass == 1) {
+      DMSC_TRY((integral_strips<32, 25>(s, g, 0, 12, frames, bands, rows, I)));
     } else {
       hipLaunchKernelGGL(k_integral_rows<32>, dim3(maxh, 12), dim3(256), (size_t)maxw, s, g, 0, frames, I);
       hipLaunchKernelGGL(k_integral_cols, dim3(div_up(maxw * 32 / 2, 256), 12), dim3(256), 0, s, g, 0, I);
     }
   }
   if (texture) {
-    if (P->band_ok && integral_pass == 1) {
-      if (tbp == 32) DMSC_TRY((integral_bands<32, 32>(s, g, 12, 4, maxw, maxh, frames, bands, I)));
-      else DMSC_TRY((integral_bands<64, 64>(s, g, 12, 4, maxw, maxh, frames, bands, I)));
+    if (integral_pass == 1) {
+      if (tbp == 32) DMSC_TRY((integral_strips<32, 32>(s, g, 12, 4, frames, bands, rows, I)));
+      else DMSC_TRY((integral_strips<64, 64>(s, g, 12, 4, frames, bands, rows, I)));
     } else {
       if (tbp == 32)
         hipLaunchKernelGGL(k_integral_rows<32>, dim3(maxh, 4), dim3(256), (size_t)maxw, s, g, 12, frames, I);

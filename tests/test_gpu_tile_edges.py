@@ -78,3 +78,20 @@ def test_spb_combine_tiles(ctx, w, h, nvec):
     gp, gp64 = host(p.grad), p64.grad.numpy()
     assert np.abs(gp - gp64).max() < (1e-5 + 2.0 * tie.sum() / n) * np.abs(gp64).max()
     assert gp[13] == 0
+
+
+# integral images: strips of 64 columns and bands of 16 rows of the rotated
+# frames (whose sides these sizes put on and off those multiples), and frames
+# wider than 2,048 columns
+@pytest.mark.parametrize("w,h,ntex", [(32, 32, 32), (68, 36, 64), (69, 133, 32), (2200, 40, 32), (40, 2100, 64)])
+def test_integral_strips(ctx, w, h, ntex):
+    print(f"case: integral strips {w}x{h}, {ntex} textons", flush=True)
+    r = np.random.RandomState(w + h)
+    L, a, b = (ctx.upload(r.rand(h, w).astype(np.float32)) for _ in range(3))
+    tex = ctx.upload(r.randint(0, ntex, (h, w)).astype(np.int32))
+    choice = dm.TEXTON64 if ntex == 64 else dm.TEXTON32
+    raws = []
+    for one_write in (0, 1):
+        with dm.tuned(integral_pass=one_write):
+            raws.append(host(ctx.local_cues(L, a, b, tex, raw=True, texton_choice=choice)[1]))
+    assert np.array_equal(bits(raws[0]), bits(raws[1]))
