@@ -364,65 +364,79 @@ struct BlurK {
   float k[16];
 };
 
+// rotate.cu:352-370: zero-padded correlation over bins.  A padding term
+// fma(0, k, s) leaves s unchanged (s >= +0, k finite), so it is not formed.
+template <int NB, int KR>
+__device__ __forceinline__ void blur_bins(float (&v)[32], const BlurK& bk) {
+  float c[NB];
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    float s = 0.f;
+#pragma unroll
+    for (int nk = 0; nk < 2 * KR + 1; nk++) {
+      const int j = i - KR + nk;
+      if (j >= 0 && j < NB) s = fmaf(v[j], bk.k[nk], s);
+    }
+    c[i] = s;
+  }
+#pragma unroll
+  for (int i = 0; i < NB; i++) v[i] = c[i];
+}
+
 // rotate.cu:263-475 computeGradient: one (pixel, scale, split) per thread.
 // NB bins, KR blur radius (0 = no blur).  Output plane of channel ch:
 // [scale][slot] with slot o+4 for the top/bottom split (sense A) and slot o
 // for the left/right split (sense B) (gradient.cu:240-241).
+// c[i0] - c[i1] + c[i2] - c[i3] of packed corner counts, two bins per word,
+// each half modulo 2^16 on its own.
+template <int NB>
+__device__ __forceinline__ void corner_sum(const uint32_t (&pk)[8][16], int i0, int i1, int i2, int i3,
+                                           uint32_t (&out)[16]) {
+#pragma unroll
+  for (int e = 0; e < 16; e++)
+    out[e] = 2 * e < NB ? __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, pk[i0][e]) -
+                                                           __builtin_bit_cast(u16x2, pk[i1][e]) +
+                                                           __builtin_bit_cast(u16x2, pk[i2][e]) -
+                                                           __builtin_bit_cast(u16x2, pk[i3][e]))
+                        : 0u;
+}
+
 // chi^2 of one split of the half-disc pair from the packed corner counts:
 // a = c[i0] - c[i1] + c[i2] - c[i3], b = c[j0] - c[j1] + c[j2] - c[j3] per
 // bin (uint16 modulo arithmetic recovers the exact counts), optional bin
 // blur, normalisation to sum 8 and 0.5 * sum (a-b)^2/(a+b) with the
 // reference's 32-slot tree sums (rotate.cu:352-472).
+// Divisions: n / s for the values that occur here (0 or n in [2^-80, 2^7], s
+// in [2^-17, 2^10]), where no scaling is needed: Newton steps with fused
+// multiply-adds from the hardware reciprocal, whose last correction rounds
+// correctly (Markstein, IBM J. Res. Dev. 34, 1990), so the quotient is the
+// IEEE one.  It saves the scaling and fix-up instructions of the general
+// sequence and leaves no branch per bin.
+__device__ __forceinline__ float div_exact(float n, float s) {
+  float r = __builtin_amdgcn_rcpf(s);
+  r = fmaf(fmaf(-s, r, 1.0f), r, r);
+  float q = n * r;
+  q = fmaf(fmaf(-s, q, n), r, q);
+  return fmaf(fmaf(-s, q, n), r, q);
+}
+
 // PAIR: the pixel's 64 bins are split over this lane (32 bins in pk) and
 // its neighbour lane (lane ^ 1); each 32-slot tree sum is completed with the
 // partner's as lo + hi (rotate.cu:384-389 adds slot 32 to slot 0), and IEEE
 // addition being commutative both lanes hold the same total.
 template <int NB, int KR, bool PAIR = false>
-__device__ __forceinline__ float chi2_split(const uint32_t (&pk)[8][16], int i0, int i1, int i2, int i3, int j0,
-                                            int j1, int j2, int j3, const BlurK& bk) {
+__device__ __forceinline__ float chi2_split(const uint32_t (&pa)[16], const uint32_t (&pb)[16],
+                                            const BlurK& bk) {
   static_assert(!PAIR || (NB == 32 && KR == 0), "paired halves hold 32 unblurred bins");
   float a[32], b[32];
-  // two bins per 32-bit word: the corner sums in packed 16-bit arithmetic,
-  // each half modulo 2^16 on its own
 #pragma unroll
-  for (int e = 0; e < 16; e++) {
-    if (2 * e < NB) {
-      const u16x2 s0 = __builtin_bit_cast(u16x2, pk[i0][e]) - __builtin_bit_cast(u16x2, pk[i1][e]) +
-                       __builtin_bit_cast(u16x2, pk[i2][e]) - __builtin_bit_cast(u16x2, pk[i3][e]);
-      const u16x2 s1 = __builtin_bit_cast(u16x2, pk[j0][e]) - __builtin_bit_cast(u16x2, pk[j1][e]) +
-                       __builtin_bit_cast(u16x2, pk[j2][e]) - __builtin_bit_cast(u16x2, pk[j3][e]);
-      a[2 * e] = (float)s0.x;
-      b[2 * e] = (float)s1.x;
-      a[2 * e + 1] = 2 * e + 1 < NB ? (float)s0.y : 0.f;
-      b[2 * e + 1] = 2 * e + 1 < NB ? (float)s1.y : 0.f;
-    } else {
-      a[2 * e] = a[2 * e + 1] = 0.f;
-      b[2 * e] = b[2 * e + 1] = 0.f;
-    }
+  for (int e = 0; e < 32; e++) {
+    a[e] = e < NB ? (float)((pa[e / 2] >> (16 * (e & 1))) & 0xffffu) : 0.f;
+    b[e] = e < NB ? (float)((pb[e / 2] >> (16 * (e & 1))) & 0xffffu) : 0.f;
   }
-  if (KR > 0) {  // rotate.cu:352-370: zero-padded correlation over bins
-    float ca[NB], cb[NB];
-#pragma unroll
-    for (int i = 0; i < NB; i++) {
-      float sa = 0.f, sb = 0.f;
-#pragma unroll
-      for (int nk = 0; nk < 2 * KR + 1; nk++) {
-        // a padding term fma(0, k, s) leaves s unchanged (s >= +0, k
-        // finite), so it is not formed
-        const int j = i - KR + nk;
-        if (j >= 0 && j < NB) {
-          sa = fmaf(a[j], bk.k[nk], sa);
-          sb = fmaf(b[j], bk.k[nk], sb);
-        }
-      }
-      ca[i] = sa;
-      cb[i] = sb;
-    }
-#pragma unroll
-    for (int i = 0; i < NB; i++) {
-      a[i] = ca[i];
-      b[i] = cb[i];
-    }
+  if constexpr (KR > 0) {
+    blur_bins<NB, KR>(a, bk);
+    blur_bins<NB, KR>(b, bk);
   }
   // slots NB..31 hold +0 and every other slot is >= +0, so the tree sums
   // skip the additions of those zeros (x + 0 = x exactly) and the chi terms
@@ -432,22 +446,20 @@ __device__ __forceinline__ float chi2_split(const uint32_t (&pk)[8][16], int i0,
   for (int i = 0; i < 32; i++) t32[i] = a[i];
   float sa = dev::tree32z<NB>(t32);
   if (PAIR) sa = sa + __shfl_xor(sa, 1, 64);
-  const float na = (sa != 0.f) ? 8.0f / sa : 0.f;
+  const float na = (sa != 0.f) ? div_exact(8.0f, sa) : 0.f;
 #pragma unroll
   for (int i = 0; i < 32; i++) t32[i] = b[i];
   float sb = dev::tree32z<NB>(t32);
   if (PAIR) sb = sb + __shfl_xor(sb, 1, 64);
-  const float nb = (sb != 0.f) ? 8.0f / sb : 0.f;
+  const float nb = (sb != 0.f) ? div_exact(8.0f, sb) : 0.f;
 #pragma unroll
   for (int i = 0; i < 32; i++) {
     float chi = 0.f;
     if (i < NB) {
       const float ai = a[i] * na, bi = b[i] * nb;
-      const float s = ai + bi;
-      if (s != 0.f) {
-        const float d = ai - bi;
-        chi = d * d / s;
-      }
+      const float s = ai + bi, d = ai - bi;
+      const float quot = div_exact(d * d, s);  // NaN for an empty bin
+      chi = s != 0.f ? quot : 0.f;
     }
     t32[i] = chi;
   }
@@ -456,27 +468,37 @@ __device__ __forceinline__ float chi2_split(const uint32_t (&pk)[8][16], int i0,
   return 0.5f * c;
 }
 
+// The pixels of a block: a 16 x 16 patch, 16 x 4 per wave.  In a rotated
+// frame a run of image pixels is a slanted line (orientation 2: a diagonal,
+// 3: nearly a column), so 64 pixels of one image row touch up to 64 cache
+// lines per corner load and use 16 bytes of each; a patch stays compact in
+// every orientation.  With runs of 64 pixels the three launches took 352 /
+// 181 / 178 us at 481x321, and take 249 / 147 / 114 us (8 x 8 per wave 251 /
+// 152 / 123, 32 x 2 274 / 154 / 134), near four fifths of the VALU issue rate.
+constexpr int GWX = 16, GPX = 16, GPY = 256 / GPX;
+
 // Both splits of one (pixel, scale, orientation): the eight corners A..H
 // are loaded once (uint16 counts, 8 bins per 16-byte load) and feed
 //   sense A (top/bottom, slot o+4): a = A-C+E-D, b = H-F+D-E
 //   sense B (left/right, slot o):   a = A-F+G-B, b = H-C+B-G
 // (rotate.cu:400-445; gradient.cu:240-241).
-// Blocks: blockIdx.x runs over (pixel block, scale) with the scale fastest,
+// Blocks: blockIdx.x runs over (patch, scale) with the scale fastest,
 // numbered XCD-aware, so each XCD handles a contiguous band of image rows at
 // all three scales and its L2 keeps the band's rotated integral rows (plus
 // the corner reach above and below) for every gather; blockIdx.y is the
 // (channel, orientation).
 template <int NB, int KR>
-__global__ __launch_bounds__(256) void k_gradients(FrameGeom g, int ch0, int rad0, const int* __restrict__ tabs,
+__global__ __launch_bounds__(256, 3) void k_gradients(FrameGeom g, int ch0, int rad0, const int* __restrict__ tabs,
                                                    const uint16_t* __restrict__ I, BlurK bk,
                                                    float* __restrict__ grads, size_t plane) {
-  const int n = g.w * g.h;
-  const int lb = dev::xcd_block(blockIdx.x, gridDim.x);
-  const int p = (lb / 3) * blockDim.x + threadIdx.x;
-  const int scale = lb % 3;
+  const int bl = dev::xcd_block(blockIdx.x, gridDim.x);
+  const int scale = bl % 3, patch = bl / 3, ntx = (g.w + GPX - 1) / GPX;
   const int ch = ch0 + (blockIdx.y >> 2), o = blockIdx.y & 3, f = ch * 4 + o;
-  if (p >= n) return;
-  const int y = p / g.w, x = p - y * g.w;
+  const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
+  const int x = (patch % ntx) * GPX + (wv % (GPX / GWX)) * GWX + ln % GWX;
+  const int y = (patch / ntx) * GPY + (wv / (GPX / GWX)) * (64 / GWX) + ln / GWX;
+  if (x >= g.w || y >= g.h) return;
+  const int p = y * g.w + x;
   const int* t = tabs + g.tab_off[o];
   const int ix = x + kBorder, iy = y + kBorder;
   const int rx = t[2 * g.bw + iy] + t[ix];
@@ -504,8 +526,13 @@ __global__ __launch_bounds__(256) void k_gradients(FrameGeom g, int ch0, int rad
     }
   }
   // corner indices: A0 B1 C2 D3 E4 F5 G6 H7
-  const float top = chi2_split<NB, KR>(pk, 0, 2, 4, 3, 7, 5, 3, 4, bk);
-  const float left = chi2_split<NB, KR>(pk, 0, 5, 6, 1, 7, 2, 1, 6, bk);
+  uint32_t ta[16], tb[16], la[16], lb[16];
+  corner_sum<NB>(pk, 0, 2, 4, 3, ta);
+  corner_sum<NB>(pk, 7, 5, 3, 4, tb);
+  corner_sum<NB>(pk, 0, 5, 6, 1, la);
+  corner_sum<NB>(pk, 7, 2, 1, 6, lb);
+  const float top = chi2_split<NB, KR>(ta, tb, bk);
+  const float left = chi2_split<NB, KR>(la, lb, bk);
   float* dst = grads + (size_t)((ch * 3 + scale) * 8) * plane + p;
   dst[(size_t)(o + 4) * plane] = top;
   dst[(size_t)o * plane] = left;
@@ -515,18 +542,18 @@ __global__ __launch_bounds__(256) void k_gradients(FrameGeom g, int ch0, int rad
 // computeGradient<64, 64, false, *>): lanes 2p and 2p+1 share pixel p,
 // holding bins 0..31 and 32..63 of every corner (integral planes 0..3 and
 // 4..7).  Output as k_gradients.
-__global__ __launch_bounds__(256) void k_gradients64(FrameGeom g, int rad0, const int* __restrict__ tabs,
+constexpr int GHX = 16, GHY = 8;  // a block's patch: four waves of 8 x 4 pixels
+__global__ __launch_bounds__(256, 3) void k_gradients64(FrameGeom g, int rad0, const int* __restrict__ tabs,
                                                      const uint16_t* __restrict__ I, float* __restrict__ grads,
                                                      size_t plane) {
-  const int n = g.w * g.h;
-  const int lb = dev::xcd_block(blockIdx.x, gridDim.x);  // (pixel block, scale), as k_gradients
-  const int gt = (lb / 3) * blockDim.x + threadIdx.x;
-  const int half = gt & 1;
-  const bool live = (gt >> 1) < n;
-  const int p = live ? (gt >> 1) : n - 1;  // both lanes of a pair agree; all lanes reach the shuffles
-  const int scale = lb % 3;
+  const int bl = dev::xcd_block(blockIdx.x, gridDim.x);  // (patch, scale), as k_gradients
+  const int scale = bl % 3, patch = bl / 3, ntx = (g.w + GHX - 1) / GHX;
   const int ch = 3, o = blockIdx.y, f = ch * 4 + o;
-  const int y = p / g.w, x = p - y * g.w;
+  const int wv = threadIdx.x >> 6, ln = (threadIdx.x & 63) >> 1, half = threadIdx.x & 1;
+  const int xx = (patch % ntx) * GHX + (wv & 1) * 8 + ln % 8, yy = (patch / ntx) * GHY + (wv >> 1) * 4 + ln / 8;
+  const bool live = xx < g.w && yy < g.h;
+  // both lanes of a pair agree; all lanes reach the shuffles
+  const int x = live ? xx : g.w - 1, y = live ? yy : g.h - 1, p = y * g.w + x;
   const int* t = tabs + g.tab_off[o];
   const int ix = x + kBorder, iy = y + kBorder;
   const int rx = t[2 * g.bw + iy] + t[ix];
@@ -549,8 +576,13 @@ __global__ __launch_bounds__(256) void k_gradients64(FrameGeom g, int rad0, cons
     }
   }
   BlurK none{};
-  const float top = chi2_split<32, 0, true>(pk, 0, 2, 4, 3, 7, 5, 3, 4, none);
-  const float left = chi2_split<32, 0, true>(pk, 0, 5, 6, 1, 7, 2, 1, 6, none);
+  uint32_t ta[16], tb[16], la[16], lb[16];
+  corner_sum<32>(pk, 0, 2, 4, 3, ta);
+  corner_sum<32>(pk, 7, 5, 3, 4, tb);
+  corner_sum<32>(pk, 0, 5, 6, 1, la);
+  corner_sum<32>(pk, 7, 2, 1, 6, lb);
+  const float top = chi2_split<32, 0, true>(ta, tb, none);
+  const float left = chi2_split<32, 0, true>(la, lb, none);
   if (live && half == 0) {
     float* dst = grads + (size_t)((ch * 3 + scale) * 8) * plane + p;
     dst[(size_t)(o + 4) * plane] = top;
@@ -558,66 +590,85 @@ __global__ __launch_bounds__(256) void k_gradients64(FrameGeom g, int rad0, cons
   }
 }
 
-// Parabola smoothing (parabola.cu:75-124 / parabola_kernel.cu:1-30) of one
-// scale of a channel group, plane z = (channel - ch0) * 8 + orientation.
-// Each thread computes QX horizontally adjacent outputs.  For every filter
-// row v (the reference's outer loop, ascending) it loads the QX + 2R tile
-// values that row needs into registers once, then runs the fully unrolled u
-// loop (inner, ascending) over the dense (2R+1)-wide row.  Taps outside the
-// ellipse have coefficient 0 and fma(x, 0, acc) == acc for finite x (acc
-// starts at +0 and can never become -0), so the sums equal the reference's
-// zero-skipping loop bit for bit; rows with no non-zero tap are skipped.
-constexpr int QX = 8, QCOLS = 16, QTX = QX * QCOLS, QTY = 16;
+// Parabola smoothing (parabola.cu:75-124 / parabola_kernel.cu:1-30) of all
+// planes of a channel group in one launch.
+// Each thread computes QX horizontally adjacent outputs from a tile staged
+// in LDS.  The filter of a radius and orientation is a list of pieces of
+// four horizontally adjacent taps, row by row (v ascending, the reference's
+// outer loop) and u ascending within a row, that cover its non-zero taps:
+// per piece a scalar load of the four coefficients and three 16-byte LDS
+// reads feed 4 QX multiply-adds.  A covered tap outside the ellipse has
+// coefficient 0 and fma(x, 0, acc) == acc for finite x (acc starts at +0 and
+// can never become -0), so the sums equal the reference's zero-skipping loop
+// bit for bit.  The ellipse (axes r and r/4) holds a fifth of its square:
+// dense rows of 2 r + 1 taps took 120 us per channel at radius 20 (481x321),
+// 330 us for all 96 planes in nine launches; the lists take 128 us in one (59 us
+// of multiply-adds, 44 us of LDS reads; staging the tile row by row, with one
+// row's loads in flight, cost another 50).
+constexpr int QX = 8, QCOLS = 16, QTX = QX * QCOLS, QTY = 32, QNT = QCOLS * QTY;
 
-template <int R>
-constexpr int q_lw() {
-  return (QTX + 2 * R + 3) / 4 * 4;  // tile row length, float4-aligned
-}
+__host__ __device__ constexpr int q_lw(int r) { return QTX - QX + 2 * r / 4 * 4 + 12; }  // tile row, floats
+__host__ __device__ constexpr int q_lh(int r) { return QTY + 2 * r; }
 
-template <int R>
-__global__ __launch_bounds__(256) void k_parabola(int w, int h, int scale, int ch0, const float* __restrict__ grads,
-                                                  size_t gplane, const float* __restrict__ coef,
-                                                  const int2* __restrict__ vrange, CueOut out, int pitch) {
+struct ParabolaJobs {
+  int n;                              // (channel, scale) pairs, largest radius first
+  int ch[12], scale[12], radius[12];
+  int first[12][8], count[12][8];     // pieces of the pair's orientations
+};
+
+__global__ __launch_bounds__(QNT) void k_parabola(int w, int h, ParabolaJobs J, const float* __restrict__ grads,
+                                                  size_t gplane, const float4* __restrict__ coef,
+                                                  const int* __restrict__ at, CueOut out, int pitch) {
   extern __shared__ float4 tile4[];
   float* tile = reinterpret_cast<float*>(tile4);
-  constexpr int LW = q_lw<R>(), LH = QTY + 2 * R, D = 2 * R + 1;
-  constexpr int SEG = (QX + 2 * R + 3) / 4 * 4;
-  const int ch = ch0 + blockIdx.z / 8, o = blockIdx.z % 8;
+  const int job = blockIdx.z >> 3, o = blockIdx.z & 7;
+  const int ch = J.ch[job], scale = J.scale[job], R = J.radius[job], LW = q_lw(R), LH = q_lh(R);
   const float* src = grads + (size_t)((ch * 3 + scale) * 8 + o) * gplane;
   const int x0 = blockIdx.x * QTX, y0 = blockIdx.y * QTY;
-  for (int i = threadIdx.x; i < LW * LH; i += 256) {
-    const int ly = i / LW, lx = i - ly * LW;
-    // tile columns past the image only feed discarded outputs: clamp into
-    // the mirrored range [0, w + 2*border) before reflecting
-    const int gx = dev::mirror(dev::clampi(x0 + lx - R + kBorder, 0, w + 2 * kBorder - 1), kBorder, w);
-    const int gy = dev::mirror(dev::clampi(y0 + ly - R + kBorder, 0, h + 2 * kBorder - 1), kBorder, h);
-    tile[i] = src[(size_t)gy * w + gx];
+  const int lane = threadIdx.x & 63;
+  // tile columns past the image only feed discarded outputs: clamp into the
+  // mirrored range [0, w + 2*border) before reflecting
+  int gx[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++)
+    gx[k] = dev::mirror(dev::clampi(x0 + lane + 64 * k - R + kBorder, 0, w + 2 * kBorder - 1), kBorder, w);
+  constexpr int kRows = 3;  // tile rows per wave whose loads are in flight together
+  for (int l0 = threadIdx.x >> 6; l0 < LH; l0 += kRows * (QNT / 64)) {
+    float t[kRows][3];
+#pragma unroll
+    for (int r = 0; r < kRows; r++) {
+      const int ly = l0 + r * (QNT / 64);
+      const int gy = dev::mirror(dev::clampi(y0 + ly - R + kBorder, 0, h + 2 * kBorder - 1), kBorder, h);
+      const float* row = src + (size_t)gy * w;
+#pragma unroll
+      for (int k = 0; k < 3; k++) t[r][k] = row[gx[k]];
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; r++) {
+      const int ly = l0 + r * (QNT / 64);
+#pragma unroll
+      for (int k = 0; k < 3; k++)
+        if (ly < LH && lane + 64 * k < LW) tile[ly * LW + lane + 64 * k] = t[r][k];
+    }
   }
   __syncthreads();
   const int tx = (threadIdx.x % QCOLS) * QX, ty = threadIdx.x / QCOLS;
-  const float* f = coef + (size_t)o * D * D;
-  const int2 vr = vrange[o];
+  const int first = J.first[job][o], last = first + J.count[job][o];
+  const float4* base = tile4 + (ty * LW + tx) / 4;
   float acc[QX];
 #pragma unroll
   for (int j = 0; j < QX; j++) acc[j] = 0.0f;
-  for (int v = vr.x; v <= vr.y; v++) {
-    const float4* rowp = reinterpret_cast<const float4*>(tile + (ty + R + v) * LW + tx);
-    float seg[SEG];
+#pragma unroll 4
+  for (int i = first; i < last; i++) {
+    const float4 c = coef[i];
+    const float4* p = base + at[i];
+    const float4 a = p[0], b = p[1], d = p[2];
+    const float seg[12] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, d.x, d.y, d.z, d.w};
+    const float cf[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
-    for (int q = 0; q < SEG / 4; q++) {
-      const float4 t = rowp[q];
-      seg[4 * q] = t.x;
-      seg[4 * q + 1] = t.y;
-      seg[4 * q + 2] = t.z;
-      seg[4 * q + 3] = t.w;
-    }
-    const float* fr = f + (v + R) * D;
+    for (int u = 0; u < 4; u++)
 #pragma unroll
-    for (int u = 0; u < D; u++) {
-      const float c = fr[u];
-#pragma unroll
-      for (int j = 0; j < QX; j++) acc[j] = fmaf(seg[j + u], c, acc[j]);
-    }
+      for (int j = 0; j < QX; j++) acc[j] = fmaf(seg[j + u], cf[u], acc[j]);
   }
   float* dst = out.p[ch] + (size_t)(scale * 8 + o) * pitch;
   const int gy = y0 + ty;
@@ -627,29 +678,24 @@ __global__ __launch_bounds__(256) void k_parabola(int w, int h, int scale, int c
       if (x0 + tx + j < w) dst[(size_t)gy * w + x0 + tx + j] = acc[j];
 }
 
-template <int R>
-size_t parabola_lds() {
-  return sizeof(float) * (size_t)q_lw<R>() * (QTY + 2 * R) + 16;
-}
-
 // ---------------------------------------------------------------- host plan
 
 struct CuePlan {
   int w = -1, h = -1;
   FrameGeom g;
   size_t lab_bytes = 0, int_elems = 0, band_elems = 0, row_words = 0;
-  int tap_stride = 0;
   int* d_tabs = nullptr;
-  float* d_coef[4] = {nullptr, nullptr, nullptr, nullptr};  // [8][2r+1][2r+1] per radius
-  int2* d_vrange[4] = {nullptr, nullptr, nullptr, nullptr};  // rows holding non-zero taps
+  // smoothing filters as pieces of four taps: coefficients, float4 offset of
+  // the piece in a tile of its radius, and [radius][orientation] ranges
+  float4* d_piece_coef = nullptr;
+  int* d_piece_at = nullptr;
+  int piece_first[4][8], piece_count[4][8];
   BlurK blur_bg, blur_cg;
   int kr_bg = 0, kr_cg = 0;
   ~CuePlan() {
     if (d_tabs) (void)hipFree(d_tabs);
-    for (int i = 0; i < 4; i++) {
-      if (d_coef[i]) (void)hipFree(d_coef[i]);
-      if (d_vrange[i]) (void)hipFree(d_vrange[i]);
-    }
+    if (d_piece_coef) (void)hipFree(d_piece_coef);
+    if (d_piece_at) (void)hipFree(d_piece_at);
   }
 };
 
@@ -718,26 +764,35 @@ int build_plan(hipStream_t s, int w, int h, int tbp, CuePlan& P) {
   P.row_words = ro;
   DMSC_HIP(hipMalloc(&P.d_tabs, sizeof(int) * tabs.size()));
   DMSC_HIP(hipMemcpy(P.d_tabs, tabs.data(), sizeof(int) * tabs.size(), hipMemcpyHostToDevice));
+  std::vector<float4> piece_coef;
+  std::vector<int> piece_at;
   for (int ri = 0; ri < 4; ri++) {
     const int r = kRadii[ri], len = 2 * r + 1;
     std::vector<float> filt((size_t)8 * len * len);
     parabola_filters(r, filt.data());
-    std::vector<int2> vr(8);
     for (int o = 0; o < 8; o++) {
-      int v0 = r + 1, v1 = -r - 1;
-      for (int v = -r; v <= r; v++)
-        for (int u = -r; u <= r; u++)
-          if (filt[(size_t)o * len * len + (v + r) * len + (u + r)] != 0.0f) {
-            v0 = std::min(v0, v);
-            v1 = std::max(v1, v);
+      P.piece_first[ri][o] = (int)piece_coef.size();
+      for (int v = 0; v < len; v++) {
+        const float* row = filt.data() + ((size_t)o * len + v) * len;
+        int u0 = len, u1 = -1;  // columns holding the row's non-zero taps
+        for (int u = 0; u < len; u++)
+          if (row[u] != 0.0f) {
+            u0 = std::min(u0, u);
+            u1 = u;
           }
-      vr[o] = make_int2(v0, v1);  // empty range (v0 > v1) if every tap is zero
+        for (int u = u0 & ~3; u <= u1; u += 4) {
+          auto tap = [&](int k) { return k < len ? row[k] : 0.0f; };
+          piece_coef.push_back(make_float4(tap(u), tap(u + 1), tap(u + 2), tap(u + 3)));
+          piece_at.push_back((v * q_lw(r) + u) / 4);
+        }
+      }
+      P.piece_count[ri][o] = (int)piece_coef.size() - P.piece_first[ri][o];
     }
-    DMSC_HIP(hipMalloc(&P.d_coef[ri], sizeof(float) * filt.size()));
-    DMSC_HIP(hipMemcpy(P.d_coef[ri], filt.data(), sizeof(float) * filt.size(), hipMemcpyHostToDevice));
-    DMSC_HIP(hipMalloc(&P.d_vrange[ri], sizeof(int2) * 8));
-    DMSC_HIP(hipMemcpy(P.d_vrange[ri], vr.data(), sizeof(int2) * 8, hipMemcpyHostToDevice));
   }
+  DMSC_HIP(hipMalloc(&P.d_piece_coef, sizeof(float4) * piece_coef.size()));
+  DMSC_HIP(hipMemcpy(P.d_piece_coef, piece_coef.data(), sizeof(float4) * piece_coef.size(), hipMemcpyHostToDevice));
+  DMSC_HIP(hipMalloc(&P.d_piece_at, sizeof(int) * piece_at.size()));
+  DMSC_HIP(hipMemcpy(P.d_piece_at, piece_at.data(), sizeof(int) * piece_at.size(), hipMemcpyHostToDevice));
   // gradient.cu:233: blur sigma = (int)(sigma * nbins) -> Bg 2, Cg 1
   memset(&P.blur_bg, 0, sizeof(BlurK));
   memset(&P.blur_cg, 0, sizeof(BlurK));
@@ -906,45 +961,45 @@ int launch_local_cues_part(Ctx* ctx, hipStream_t s, int part, int w, int h, cons
     }
   }
   const size_t plane = (size_t)n;
+  const int patches = div_up(w, GPX) * div_up(h, GPY);
   BlurK none;
   memset(&none, 0, sizeof(none));
   // Bg: channel 0, radii {3,5,10}; Cga/Cgb: channels 1-2, radii {5,10,20};
   // Tg: channel 3, radii {5,10,20}.
   if (colour) {
-    hipLaunchKernelGGL((k_gradients<25, 6>), dim3(div_up(n, 256) * 3, 4), dim3(256), 0, s, g, 0, 0,
+    hipLaunchKernelGGL((k_gradients<25, 6>), dim3(patches * 3, 4), dim3(256), 0, s, g, 0, 0,
                        P->d_tabs, I, P->blur_bg, grads, plane);
-    hipLaunchKernelGGL((k_gradients<25, 3>), dim3(div_up(n, 256) * 3, 8), dim3(256), 0, s, g, 1, 1,
+    hipLaunchKernelGGL((k_gradients<25, 3>), dim3(patches * 3, 8), dim3(256), 0, s, g, 1, 1,
                        P->d_tabs, I, P->blur_cg, grads, plane);
   }
   if (texture) {
     if (ntex == 64)
-      hipLaunchKernelGGL(k_gradients64, dim3(div_up(2 * n, 256) * 3, 4), dim3(256), 0, s, g, 1, P->d_tabs, I,
+      hipLaunchKernelGGL(k_gradients64, dim3(div_up(w, GHX) * div_up(h, GHY) * 3, 4), dim3(256), 0, s, g, 1, P->d_tabs, I,
                          grads, plane);
     else
-      hipLaunchKernelGGL((k_gradients<32, 0>), dim3(div_up(n, 256) * 3, 4), dim3(256), 0, s, g, 3, 1,
+      hipLaunchKernelGGL((k_gradients<32, 0>), dim3(patches * 3, 4), dim3(256), 0, s, g, 3, 1,
                          P->d_tabs, I, none, grads, plane);
   }
   if (hist_done) DMSC_HIP(hipEventRecord(hist_done, s));
   CueOut out{{bg, cga, cgb, tg}};
-  for (int scale = 0; scale < 3; scale++) {
-    // (first channel, channels, radius index): Bg; Cga and Cgb; Tg
-    const int groups[3][3] = {{0, 1, scale}, {1, 2, scale + 1}, {3, 1, scale + 1}};
-    for (int gi = 0; gi < 3; gi++) {
-      if ((gi < 2 && !colour) || (gi == 2 && !texture)) continue;
-      const int ch0 = groups[gi][0], nch = groups[gi][1], ri = groups[gi][2];
-      const dim3 grid(div_up(w, QTX), div_up(h, QTY), nch * 8);
-      switch (kRadii[ri]) {
-#define PARABOLA_CASE(R)                                                                                   \
-  case R:                                                                                                  \
-    hipLaunchKernelGGL(k_parabola<R>, grid, dim3(256), parabola_lds<R>(), s, w, h, scale, ch0, grads,       \
-                       plane, P->d_coef[ri], P->d_vrange[ri], out, pitch);                                \
-    break;
-        PARABOLA_CASE(3) PARABOLA_CASE(5) PARABOLA_CASE(10) PARABOLA_CASE(20)
-#undef PARABOLA_CASE
-        default: return fail(DMSC_ERR_INTERNAL, "no parabola kernel for radius %d", kRadii[ri]);
-      }
+  ParabolaJobs J;
+  J.n = 0;
+  for (int ri = 3; ri >= 0; ri--)  // longest blocks first
+    for (int ch = 0; ch < 4; ch++) {
+      const int scale = ri - (ch == 0 ? 0 : 1);  // Bg: radii 3, 5, 10; the others 5, 10, 20
+      if (scale < 0 || scale > 2 || (ch < 3 ? !colour : !texture)) continue;
+      J.ch[J.n] = ch;
+      J.scale[J.n] = scale;
+      J.radius[J.n] = kRadii[ri];
+      std::copy(P->piece_first[ri], P->piece_first[ri] + 8, J.first[J.n]);
+      std::copy(P->piece_count[ri], P->piece_count[ri] + 8, J.count[J.n]);
+      J.n++;
     }
-  }
+  static_assert(q_lw(3) % 4 == 0 && q_lw(5) % 4 == 0 && q_lw(10) % 4 == 0 && q_lw(20) % 4 == 0 && q_lw(20) <= 192,
+                "float4-aligned tile rows of at most three columns per lane");
+  hipLaunchKernelGGL(k_parabola, dim3(div_up(w, QTX), div_up(h, QTY), J.n * 8), dim3(QNT),
+                     sizeof(float) * q_lw(J.radius[0]) * q_lh(J.radius[0]), s, w, h, J, grads, plane, P->d_piece_coef,
+                     P->d_piece_at, out, pitch);
   DMSC_HIP(hipGetLastError());
   return DMSC_OK;
 }

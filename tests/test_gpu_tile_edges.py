@@ -95,3 +95,20 @@ def test_integral_strips(ctx, w, h, ntex):
         with dm.tuned(integral_pass=one_write):
             raws.append(host(ctx.local_cues(L, a, b, tex, raw=True, texton_choice=choice)[1]))
     assert np.array_equal(bits(raws[0]), bits(raws[1]))
+
+
+# gradients in 16 x 16 patches (32 textons and the L/a/b bins) and 16 x 8 ones
+# (64 textons), smoothing in tiles of 128 x 32 outputs: partial tiles on both
+# sides, against the oracle
+@pytest.mark.parametrize("w,h,ntex", [(32, 33, 32), (129, 47, 32), (127, 65, 64), (144, 64, 64)])
+def test_local_cues_tiles(ctx, w, h, ntex):
+    print(f"case: local cues {w}x{h}, {ntex} textons", flush=True)
+    r = np.random.RandomState(3 * w + h)
+    L, a, b = (np.clip(r.rand(h, w) * 1.1 - 0.05, 0, 1).astype(np.float32) for _ in range(3))
+    tex = r.randint(0, ntex, (h, w)).astype(np.int32)
+    tex[h // 3:, w // 2:] = 1  # flat regions: empty bins on both sides of a split
+    a[:, w // 2:] = 0.5
+    got = ctx.local_cues(*[ctx.upload(v) for v in (L, a, b)], ctx.upload(tex),
+                         texton_choice=dm.TEXTON64 if ntex == 64 else dm.TEXTON32)
+    for c, ref in zip(got, O.local_cues(L, a, b, tex, ntex=ntex)):
+        assert np.array_equal(bits(host(c)), bits(np.asarray(ref).reshape(24, -1)[:, :w * h]))
