@@ -481,14 +481,8 @@ int dmsc_kmeans(dmsc_ctx* ctx, int w, int h, int k, int nfilters, const float* r
   DMSC_ARG(precision == DMSC_PREC_FP32 || precision == DMSC_PREC_MIXED, "bad precision");
   const int n = w * h;
   void* scr;
-  const size_t st = (kmeans_state_bytes() + 255) & ~(size_t)255;
-  DMSC_TRY(ctx->scratch(2, st + sizeof(float) * (size_t)pitch_floats(n), &scr));
-  float* pdot = (float*)((char*)scr + st);
-  if (precision == DMSC_PREC_MIXED) {
-    DMSC_TRY(launch_kmeans_mixed(ctx->stream, w, h, k, resp, labels, pdot, scr, max_iter));
-  } else {
-    DMSC_TRY(launch_kmeans(ctx->stream, w, h, k, nfilters, resp, labels, pdot, scr, max_iter));
-  }
+  DMSC_TRY(ctx->scratch(2, kmeans_state_bytes(), &scr));
+  DMSC_TRY(launch_kmeans(ctx->stream, w, h, k, resp, labels, scr, max_iter));
   return kmeans_read_state(ctx->stream, scr, changes, iterations);
 }
 
@@ -496,7 +490,8 @@ int dmsc_kmeans_rechecks(dmsc_ctx* ctx, int* rechecks) {
   CHECK_CTX(ctx);
   DMSC_ARG(rechecks, "null pointer");
   DMSC_ARG(ctx->arena[2] && ctx->arena_bytes[2] >= kmeans_state_bytes(), "no k-means run on this context");
-  return kmeans_read_state(ctx->stream, ctx->arena[2], nullptr, nullptr, rechecks);
+  *rechecks = 0;  // the distances are exact: no assignment is ever recomputed
+  return DMSC_OK;
 }
 
 int dmsc_eigensolve_report(dmsc_ctx* ctx, int* stop_rule, double* max_residual) {
@@ -831,13 +826,8 @@ int dmsc_gpb(dmsc_ctx* ctx, int w, int h, const uint32_t* rgb, const dmsc_gpb_pa
   if (timing) DMSC_HIP(hipEventRecord(ev[7], s));
   {
     void* scr;
-    const size_t st = (kmeans_state_bytes() + 255) & ~(size_t)255;
-    DMSC_TRY(ctx->scratch(2, st + sizeof(float) * P, &scr));
-    float* pdot = (float*)((char*)scr + st);
-    if (p.precision == DMSC_PREC_MIXED)
-      DMSC_TRY(launch_kmeans_mixed(s, w, h, ntex, resp, tex, pdot, scr, 15));
-    else
-      DMSC_TRY(launch_kmeans(s, w, h, ntex, kNFilters, resp, tex, pdot, scr, 15));
+    DMSC_TRY(ctx->scratch(2, kmeans_state_bytes(), &scr));
+    DMSC_TRY(launch_kmeans(s, w, h, ntex, resp, tex, scr, 15));
     // the iteration count reaches the host without a stream synchronisation
     // here: the eigensolver synchronises before it returns
     DMSC_TRY(ctx->pinned(&kit));

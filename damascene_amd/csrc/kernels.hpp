@@ -19,11 +19,9 @@ int launch_quantize(hipStream_t s, int n, int nbins, const float* in, int* out);
 // ------------------------------------------------------------- textons
 int launch_texton_conv(hipStream_t s, int w, int h, const float* grey, const float* d_coeffs, float* resp);
 size_t kmeans_state_bytes();
-int launch_kmeans(hipStream_t s, int w, int h, int k, int nf, const float* resp, int* labels, float* pdot,
-                  void* state, int max_iter);
-int launch_kmeans_mixed(hipStream_t s, int w, int h, int k, const float* resp, int* labels, float* pdot,
-                        void* state, int max_iter);
-int kmeans_read_state(hipStream_t s, void* state, int* changes, int* iterations, int* rechecks = nullptr);
+// Exact FP32 distances at either precision (the labels are the same).
+int launch_kmeans(hipStream_t s, int w, int h, int k, const float* resp, int* labels, void* state, int max_iter);
+int kmeans_read_state(hipStream_t s, const void* state, int* changes, int* iterations);
 const int* kmeans_iterations_ptr(const void* state);  // device address of the iteration count
 // Device address of the current device's copy of the fixed k-means scratch
 // of dmsc_kmeans_noalloc (looked up once per device; `device` is current).

@@ -1,9 +1,9 @@
 // noalloc.hip -- a k-means entry point that allocates no device memory.
 //
 // dmsc_kmeans_noalloc runs the same kernels as dmsc_kmeans (textons.hip),
-// with their scratch (the k-means state and the per-pixel |x|^2) carved out
-// of one file-scope device array instead of the context's grow-only arenas
-// (8 MiB: about 2.09 million pixels, a 1920 x 1080 image fits).  Each
+// with their scratch (the k-means state) in one file-scope device array
+// instead of the context's grow-only arenas (8 MiB; inputs of up to about 2.09
+// million pixels, a 1920 x 1080 image fits).  Each
 // GPU holds its own copy of the array from the time the library's code
 // object is loaded until the process ends.  In host code `scratch` names a
 // host-side stand-in, not device memory: the device address of each GPU's
@@ -26,11 +26,9 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
 
-size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
-
-// Scratch bytes a call over n pixels needs: the state and |x|^2 per pixel
-// (pitch_floats(n) floats); both precisions need the same.
-size_t noalloc_need(long n) { return round256(kmeans_state_bytes()) + sizeof(float) * (size_t)pitch_floats(n); }
+// The largest input: what the array held when |x|^2 was kept per pixel, and
+// the documented limit.  The k-means state alone is needed now.
+constexpr long kMaxPixels = 2092608;
 
 }  // namespace
 
@@ -56,13 +54,7 @@ using namespace dmsc;
 extern "C" {
 
 size_t dmsc_kmeans_noalloc_max_pixels(void) {
-  long lo = 0, hi = (1L << 28) - 1;  // largest n with noalloc_need(n) <= kScratchBytes
-  while (lo < hi) {
-    const long mid = (lo + hi + 1) / 2;
-    if (noalloc_need(mid) <= kScratchBytes) lo = mid;
-    else hi = mid - 1;
-  }
-  return (size_t)lo;
+  return (size_t)kMaxPixels;
 }
 
 int dmsc_kmeans_noalloc(dmsc_ctx* ctx, int w, int h, int k, int nfilters, const float* resp, int* labels,
@@ -74,21 +66,14 @@ int dmsc_kmeans_noalloc(dmsc_ctx* ctx, int w, int h, int k, int nfilters, const 
   DMSC_ARG(conv_thresh == 0, "only conv_thresh=0 (the reference default) is supported");
   DMSC_ARG(precision == DMSC_PREC_FP32 || precision == DMSC_PREC_MIXED, "bad precision");
   const long n = (long)w * h;
-  DMSC_ARG(n < (1L << 28) && noalloc_need(n) <= kScratchBytes,
-           "%dx%d needs %zu bytes of k-means scratch; the fixed scratch holds %zu (at most %zu pixels)", w, h,
-           noalloc_need(n < (1L << 28) ? n : 0), kScratchBytes, dmsc_kmeans_noalloc_max_pixels());
+  DMSC_ARG(n <= kMaxPixels, "%dx%d has %ld pixels; the fixed scratch serves at most %ld", w, h, n, kMaxPixels);
+  if (kmeans_state_bytes() > kScratchBytes) return fail(DMSC_ERR_INTERNAL, "k-means state exceeds the fixed scratch");
   DMSC_HIP(hipSetDevice(ctx->device));
   void* base = nullptr;
   DMSC_TRY(noalloc_scratch_init(ctx->device, &base));
-  char* state = (char*)base;
-  float* pdot = (float*)(state + round256(kmeans_state_bytes()));
-  if (precision == DMSC_PREC_MIXED) {
-    DMSC_TRY(launch_kmeans_mixed(ctx->stream, w, h, k, resp, labels, pdot, state, max_iter));
-  } else {
-    DMSC_TRY(launch_kmeans(ctx->stream, w, h, k, nfilters, resp, labels, pdot, state, max_iter));
-  }
+  DMSC_TRY(launch_kmeans(ctx->stream, w, h, k, resp, labels, base, max_iter));
   if (!changes && !iterations) return DMSC_OK;  // enqueued only; no read-back, no synchronisation
-  return kmeans_read_state(ctx->stream, state, changes, iterations);
+  return kmeans_read_state(ctx->stream, base, changes, iterations);
 }
 
 }  // extern "C"

@@ -111,21 +111,19 @@ int dmsc_quantize_image(dmsc_ctx* ctx, int w, int h, int nbins, const float* d_i
 int dmsc_texton_responses(dmsc_ctx* ctx, int w, int h, const float* d_grey, float* d_resp);
 /* kmeans.h:18 kmeans: k=32 or 64 clusters over [nfilters][N] responses; labels
  * out; *changes = label changes of the last iteration; *iterations = count.
- * precision: DMSC_PREC_FP32 (VALU distances, reference order) or
- * DMSC_PREC_MIXED (BF16 MFMA distances + FP32 re-check of near ties; same
- * labels). */
+ * Both precisions take the exact FP32 distances (on the matrix cores, in the
+ * reference's order), so the labels are the same. */
 int dmsc_kmeans(dmsc_ctx* ctx, int w, int h, int k, int nfilters, const float* d_resp,
                 int* d_labels, int max_iter, int conv_thresh, int precision, int* changes,
                 int* iterations);
-/* No reference counterpart: after a DMSC_PREC_MIXED dmsc_kmeans call on this
- * context, the number of pixel assignments (summed over iterations) whose
- * BF16 MFMA distances could not certify the winner and were recomputed with
- * the exact FP32 distances. */
+/* No reference counterpart: after a dmsc_kmeans call on this context, the
+ * number of pixel assignments whose distances had to be recomputed exactly:
+ * 0, since the distances of both precisions are exact. */
 int dmsc_kmeans_rechecks(dmsc_ctx* ctx, int* rechecks);
 /* No reference counterpart: dmsc_kmeans for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, kernels and labels as
- * dmsc_kmeans; its scratch (the k-means state and |x|^2 per pixel) lives in
+ * dmsc_kmeans; its scratch (the k-means state) lives in
  * a fixed device array of DMSC_KMEANS_NOALLOC_SCRATCH_BYTES per GPU, held
  * from library load to process exit, so the call allocates nothing.  Inputs
  * of more than dmsc_kmeans_noalloc_max_pixels() pixels (2,092,608: a

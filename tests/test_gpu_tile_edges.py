@@ -112,3 +112,22 @@ def test_local_cues_tiles(ctx, w, h, ntex):
                          texton_choice=dm.TEXTON64 if ntex == 64 else dm.TEXTON32)
     for c, ref in zip(got, O.local_cues(L, a, b, tex, ntex=ntex)):
         assert np.array_equal(bits(host(c)), bits(np.asarray(ref).reshape(24, -1)[:, :w * h]))
+
+
+# k-means: 256-pixel chunks, up to 768 looping blocks, 32 clusters per pass of
+# the matrix cores; ties and empty clusters
+@pytest.mark.parametrize("w,h,k", [(7, 5, 32), (16, 16, 64), (257, 3, 32), (515, 397, 64), (900, 700, 32)])
+def test_kmeans_chunks(ctx, w, h, k):
+    print(f"case: k-means {w}x{h}, {k} clusters", flush=True)
+    r = np.random.RandomState(w + k)
+    resp = (r.randn(34, h, w) * 0.1).astype(np.float32)
+    resp[:, : h // 2, : w // 3] = 0.0  # equal pixels: equal distances
+    resp[33] = 0.0
+    labels, it = ctx.kmeans(ctx.upload(resp), k=k)
+    ref, rit = O.kmeans(resp, k=k)
+    assert it == rit
+    np.testing.assert_array_equal(host(labels), ref)
+    # a pixel whose squared distance to every centroid passes 1e7 gets no label
+    resp[5, h - 1, w - 1] = 30000.0 if w * h > 1000 else 0.0
+    far, _ = ctx.kmeans(ctx.upload(resp), k=k, max_iter=1)
+    assert int((far < 0).sum()) == (1 if w * h > 1000 else 0) and (w * h <= 1000 or far[h - 1, w - 1] == -1)
