@@ -98,9 +98,9 @@ int Ctx::adopt(int slot, void* p, size_t bytes) {
 
 int Ctx::texton_coeffs(const float** out) {
   if (!d_texton_coeffs) {
-    const TextonBank& b = texton_bank();
-    DMSC_HIP(hipMalloc(&d_texton_coeffs, sizeof(float) * b.coeffs.size()));
-    DMSC_HIP(hipMemcpy(d_texton_coeffs, b.coeffs.data(), sizeof(float) * b.coeffs.size(), hipMemcpyHostToDevice));
+    const std::vector<float> t = texton_taps();
+    DMSC_HIP(hipMalloc(&d_texton_coeffs, sizeof(float) * t.size()));
+    DMSC_HIP(hipMemcpy(d_texton_coeffs, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice));
   }
   *out = d_texton_coeffs;
   return DMSC_OK;

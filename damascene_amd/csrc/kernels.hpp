@@ -17,7 +17,8 @@ int launch_unmirror_f(hipStream_t s, int bw, int bh, int border, const float* in
 int launch_quantize(hipStream_t s, int n, int nbins, const float* in, int* out);
 
 // ------------------------------------------------------------- textons
-int launch_texton_conv(hipStream_t s, int w, int h, const float* grey, const float* d_coeffs, float* resp);
+std::vector<float> texton_taps();  // the bank's taps as launch_texton_conv reads them
+int launch_texton_conv(hipStream_t s, int w, int h, const float* grey, const float* d_taps, float* resp);
 size_t kmeans_state_bytes();
 // Exact FP32 distances at either precision (the labels are the same).
 int launch_kmeans(hipStream_t s, int w, int h, int k, const float* resp, int* labels, void* state, int max_iter);

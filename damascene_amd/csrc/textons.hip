@@ -2,11 +2,8 @@
 // textons/kmeans.cu).
 //
 // Filter bank: exact FP32 correlation in the reference order (x offset
-// outer, y offset inner, fused multiply-add), clamp-to-edge borders.  Each
-// block stages a clamped image tile with halo in LDS; each thread computes 8
-// vertically adjacent outputs so one column of tile values feeds 8
-// independent accumulation chains.  Coefficients are wave-uniform (scalar
-// loads).
+// outer, y offset inner, fused multiply-add), clamp-to-edge borders, on the
+// matrix cores.
 //
 // k-means: one kernel per iteration.  Every block forms the centroids from
 // the int32 sums in LDS while its pixels' responses load, takes the 32 or 64
@@ -24,53 +21,95 @@
 namespace dmsc {
 namespace {
 
-constexpr int TX = 64, TY = 32, RPT = 8;  // tile 64 x 32, 8 rows per thread
+// The bank's filters 0..16 have radius 6 and 17..32 radius 9 (filter 33 is
+// zero).  v_mfma_f32_16x16x1_4b_f32 adds four blocks of a 16 x 16 outer product
+// with one step of k: row i is filter i of a scale, a column one of the wave's
+// 64 pixels (block l / 16, lane l its own pixel's value), so 16 filters of 64
+// pixels advance by one tap and every sum is the reference's fmaf chain.  A
+// block takes 64 x 4 RW pixels, RW rows per wave; its grey tile and the 16
+// filters' taps lie in LDS.  The 17th filter of radius 6 runs on the vector
+// units beside them.  One filter per block and 8 pixels per thread took 28 +
+// 45 us at 481x321 (88 + 155 us at 1024x768); one launch of both scales takes
+// 38 us (136 us), of which the MFMAs are 18 (85) and the responses' stores,
+// 21 MB (107 MB), most of the rest.
+constexpr int TX = 64;
+constexpr int kRows16 = 16;  // filters on the matrix cores
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-template <int R>
-__global__ __launch_bounds__(256) void k_texton_conv(int w, int h, const float* __restrict__ grey,
-                                                     const float* __restrict__ coeffs,
-                                                     int first_filter, float* __restrict__ out) {
-  constexpr int LW = TX + 2 * R, LH = TY + 2 * R, D = 2 * R + 1;
-  __shared__ float tile[LH][LW + 1];
-  const int f = first_filter + blockIdx.z;
+constexpr int kTaps9 = 19 * 19 * kRows16, kTaps6 = 13 * 13 * kRows16;
+template <int R, int RW>
+constexpr int bank_lds() {  // floats: the tile and the taps
+  return (TX + 2 * R) * (4 * RW + 2 * R) + (2 * R + 1) * (2 * R + 1) * kRows16;
+}
+
+template <int R, int RW, bool ODD>
+__device__ __forceinline__ void texton_bank(float* lds, int w, int h, const float* __restrict__ grey,
+                                            const float* __restrict__ bank, const float* __restrict__ odd,
+                                            float* __restrict__ out) {
+  constexpr int LW = TX + 2 * R, TY = 4 * RW, LH = TY + 2 * R, D = 2 * R + 1;
+  float* taps = lds;  // [dx][dy][filter]
+  float* tile = lds + D * D * kRows16;
   const int x0 = blockIdx.x * TX, y0 = blockIdx.y * TY;
   for (int i = threadIdx.x; i < LW * LH; i += 256) {
     const int ly = i / LW, lx = i - ly * LW;
     const int gx = dev::clampi(x0 + lx - R, 0, w - 1), gy = dev::clampi(y0 + ly - R, 0, h - 1);
-    tile[ly][lx] = grey[(size_t)gy * w + gx];
+    tile[i] = grey[(size_t)gy * w + gx];
   }
+  for (int i = threadIdx.x; i < D * D * kRows16 / 4; i += 256)
+    reinterpret_cast<float4*>(taps)[i] = reinterpret_cast<const float4*>(bank)[i];
   __syncthreads();
-  const int tx = threadIdx.x & 63, ty = (threadIdx.x >> 6) * RPT;
-  const float* c = coeffs + (size_t)(f < 17 ? f * 169 : 17 * 169 + (f - 17) * 361);
-  float acc[RPT];
+  const int lane = threadIdx.x & 63, ty = (threadIdx.x >> 6) * RW;
+  const float* col = tile + ty * LW + lane;
+  const float* tap = taps + (lane & 15);
+  f32x16 acc[RW];
+  float acc_odd[RW];
 #pragma unroll
-  for (int k = 0; k < RPT; k++) acc[k] = 0.0f;
+  for (int k = 0; k < RW; k++) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[k][r] = 0.0f;
+    acc_odd[k] = 0.0f;
+  }
 #pragma unroll 1
   for (int dx = 0; dx < D; dx++) {
-    float col[RPT + 2 * R];
+    float v[D + RW - 1], a[D];
 #pragma unroll
-    for (int j = 0; j < RPT + 2 * R; j++) col[j] = tile[ty + j][tx + dx];
+    for (int dy = 0; dy < D; dy++) a[dy] = tap[(dx * D + dy) * kRows16];
 #pragma unroll
-    for (int dy = 0; dy < D; dy++) {
-      const float cf = c[dx * D + dy];
+    for (int j = 0; j < D + RW - 1; j++) v[j] = col[j * LW + dx];
 #pragma unroll
-      for (int k = 0; k < RPT; k++) acc[k] = fmaf(col[k + dy], cf, acc[k]);
-    }
+    for (int dy = 0; dy < D; dy++)
+#pragma unroll
+      for (int k = 0; k < RW; k++) {
+        acc[k] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[dy], v[dy + k], acc[k], 0, 0, 0);
+        if (ODD) acc_odd[k] = fmaf(v[dy + k], odd[dx * D + dy], acc_odd[k]);
+      }
   }
-  const int gx = x0 + tx;
-  if (gx < w) {
-    const size_t n = (size_t)w * h;
+  const size_t n = (size_t)w * h;
 #pragma unroll
-    for (int k = 0; k < RPT; k++) {
-      const int gy = y0 + ty + k;
-      if (gy < h) out[(size_t)f * n + (size_t)gy * w + gx] = acc[k];
+  for (int k = 0; k < RW; k++) {
+    const int y = y0 + ty + k;
+    if (y >= h) continue;
+    const size_t row = (size_t)y * w;
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      const int x = x0 + 16 * b + (lane & 15);
+      if (x < w)
+#pragma unroll
+        for (int r = 0; r < 4; r++) out[(size_t)(4 * (lane >> 4) + r) * n + row + x] = acc[k][4 * b + r];
     }
+    // the odd filter of this scale; the last plane of the bank is zero
+    if (x0 + lane < w) out[(size_t)kRows16 * n + row + x0 + lane] = ODD ? acc_odd[k] : 0.0f;
   }
 }
 
-__global__ void k_zero(float* p, size_t n) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0f;
+template <int RW>
+__global__ __launch_bounds__(256) void k_texton_bank(int w, int h, const float* __restrict__ grey,
+                                                     const float* __restrict__ taps, float* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) float lds[bank_lds<9, RW>()];
+  if (blockIdx.z == 0)  // the longer blocks first
+    texton_bank<9, RW, false>(lds, w, h, grey, taps, nullptr, out + (size_t)17 * w * h);
+  else
+    texton_bank<6, RW, true>(lds, w, h, grey, taps + kTaps9, taps + kTaps9 + kTaps6, out);
 }
 
 // ------------------------------------------------------------------ k-means
@@ -304,13 +343,32 @@ __global__ __launch_bounds__(256, 3) void k_km_pass(int n, const float* __restri
 
 }  // namespace
 
-int launch_texton_conv(hipStream_t s, int w, int h, const float* grey, const float* d_coeffs, float* resp) {
-  dim3 grid(div_up(w, TX), div_up(h, TY), 17);
-  hipLaunchKernelGGL(k_texton_conv<6>, grid, dim3(256), 0, s, w, h, grey, d_coeffs, 0, resp);
-  grid.z = 16;
-  hipLaunchKernelGGL(k_texton_conv<9>, grid, dim3(256), 0, s, w, h, grey, d_coeffs, 17, resp);
-  const size_t n = (size_t)w * h;
-  hipLaunchKernelGGL(k_zero, dim3(div_up(n, 256)), dim3(256), 0, s, resp + 33 * n, n);
+// Taps of radius 9's 16 filters, radius 6's first 16 ([tap][filter] each,
+// tap = dx (2 R + 1) + dy) and radius 6's last one.
+std::vector<float> texton_taps() {
+  const TextonBank& b = texton_bank();
+  std::vector<float> t;
+  t.reserve(kTaps9 + kTaps6 + 169);
+  for (int i = 0; i < 361; i++)
+    for (int f = 0; f < kRows16; f++) t.push_back(b.coeffs[17 * 169 + (size_t)f * 361 + i]);
+  for (int i = 0; i < 169; i++)
+    for (int f = 0; f < kRows16; f++) t.push_back(b.coeffs[(size_t)f * 169 + i]);
+  for (int i = 0; i < 169; i++) t.push_back(b.coeffs[(size_t)kRows16 * 169 + i]);
+  return t;
+}
+
+int launch_texton_conv(hipStream_t s, int w, int h, const float* grey, const float* d_taps, float* resp) {
+  // two rows per wave halve the reads of the taps and the tile's frame, and
+  // pay once the grid is several rounds deep (1024x768, 3,072 blocks: 136
+  // against 147 us); at 481x321 (656 blocks, fewer than the chip holds) one
+  // row per wave balances better (38 against 42 us)
+  const int blocks2 = div_up(w, TX) * div_up(h, 8) * 2;
+  if (blocks2 >= 2048)
+    hipLaunchKernelGGL(k_texton_bank<2>, dim3(div_up(w, TX), div_up(h, 8), 2), dim3(256), 0, s, w, h, grey, d_taps,
+                       resp);
+  else
+    hipLaunchKernelGGL(k_texton_bank<1>, dim3(div_up(w, TX), div_up(h, 4), 2), dim3(256), 0, s, w, h, grey, d_taps,
+                       resp);
   DMSC_HIP(hipGetLastError());
   return DMSC_OK;
 }

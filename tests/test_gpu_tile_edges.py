@@ -131,3 +131,12 @@ def test_kmeans_chunks(ctx, w, h, k):
     resp[5, h - 1, w - 1] = 30000.0 if w * h > 1000 else 0.0
     far, _ = ctx.kmeans(ctx.upload(resp), k=k, max_iter=1)
     assert int((far < 0).sum()) == (1 if w * h > 1000 else 0) and (w * h <= 1000 or far[h - 1, w - 1] == -1)
+
+
+# filter bank: blocks of 64 x 4 pixels (one row per wave), and of 64 x 8 from
+# 2,048 blocks on
+@pytest.mark.parametrize("w,h", [(1, 1), (64, 4), (65, 9), (130, 7), (1025, 481)])
+def test_texton_bank_tiles(ctx, w, h):
+    print(f"case: filter bank {w}x{h}", flush=True)
+    grey = np.random.RandomState(w + h).rand(h, w).astype(np.float32)
+    assert np.array_equal(bits(host(ctx.texton_responses(ctx.upload(grey)))), bits(O.texton_responses(grey)))
