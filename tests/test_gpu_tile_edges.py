@@ -140,3 +140,29 @@ def test_texton_bank_tiles(ctx, w, h):
     print(f"case: filter bank {w}x{h}", flush=True)
     grey = np.random.RandomState(w + h).rand(h, w).astype(np.float32)
     assert np.array_equal(bits(host(ctx.texton_responses(ctx.upload(grey)))), bits(O.texton_responses(grey)))
+
+
+# affinities: 64 x 4 pixel blocks; waves without a clipped window within reach
+# take the compiled walks, the others the table (another one below 11 pixels a
+# side); then L_sym
+@pytest.mark.parametrize("w,h", [(6, 6), (7, 10), (11, 11), (10, 40), (23, 21), (84, 24), (150, 45)])
+def test_affinity_windows(ctx, w, h):
+    print(f"case: affinity {w}x{h}", flush=True)
+    r = np.random.RandomState(w * h)
+    pb = np.where(r.rand(h, w) < 0.4, r.rand(h, w), 0.0).astype(np.float32)
+    pb[r.rand(h, w) < 0.05] = -0.3  # below 0: as nothing crossed
+    m = ctx.intervene(ctx.upload(pb))
+    ref = O.intervene(pb)
+    n = w * h
+    got = host(m)
+    assert np.array_equal(bits(got[:, :n]), bits(np.asarray(ref).reshape(81, -1)[:, :n]))
+    assert np.all(got[:, n:] == 0)
+    d, rs = ctx.convert_matrix(w, h, m)
+    d64 = np.zeros(n)
+    for k, (dy, dx) in enumerate((y, x) for y in range(-5, 6) for x in range(-5, 6) if y * y + x * x <= 25):
+        col = np.arange(n) + dy * w + dx
+        d64 += np.where((col >= 0) & (col < n), got[k, :n], 0.0)
+    assert np.allclose(host(d).ravel(), d64, rtol=81 * 2.0 ** -24, atol=0)
+    assert np.allclose(host(rs).ravel(), 1 / np.sqrt(d64), rtol=82 * 2.0 ** -24, atol=0)
+    L = host(m)[:, :n]
+    assert np.allclose(L[40], (d64 - got[40, :n]) / d64, rtol=0, atol=82 * 2.0 ** -24)
