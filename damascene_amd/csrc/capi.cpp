@@ -234,6 +234,11 @@ int dmsc_tune_set(const char* key, int value) {
     lanczos_k1_threads = value;
     return DMSC_OK;
   }
+  if (!std::strcmp(key, "lanczos_run_polls")) {
+    DMSC_ARG(value >= 0 && value <= 1 << 20, "lanczos_run_polls must be in [0, 2^20]");
+    lanczos_run_polls = value;
+    return DMSC_OK;
+  }
   if (!std::strcmp(key, "lanczos_mixed_fused")) {
     DMSC_ARG(value >= 0 && value <= 2, "lanczos_mixed_fused must be 0, 1 or 2");
     lanczos_mixed_fused = value;
@@ -332,6 +337,10 @@ int dmsc_tune_get(const char* key, int* value) {
   }
   if (!std::strcmp(key, "lanczos_mixed_stop")) {
     *value = lanczos_mixed_stop;
+    return DMSC_OK;
+  }
+  if (!std::strcmp(key, "lanczos_run_polls")) {
+    *value = lanczos_run_polls;
     return DMSC_OK;
   }
   if (!std::strcmp(key, "lanczos_check_max")) {

@@ -19,7 +19,9 @@
 //    images at a subspace error of 1.7e-4, tol * 1e-4 kept all three
 //    below 2.1e-5).
 //
-// A plain step is two kernels and no host round trip:
+// A plain step on images of up to kRunRows rows per compute unit runs inside
+// one launch per check (k_lz_run).  Otherwise it is two kernels, with no host
+// round trip either:
 //   K1: beta_{k-1} from the |z|^2 partials (every block reduces them in the
 //       same order, so all blocks agree bit for bit), q_k = z_{k-1}/beta_{k-1}
 //       formed on the fly for the stencil gather and written to the basis,
@@ -60,6 +62,7 @@ int lanczos_max_iter = kMaxIter;
 int lanczos_check_max = 0;
 int lanczos_mixed_stop = 4;
 int lanczos_step_loads = 0;
+int lanczos_run_polls = 1 << 14;
 
 namespace {
 
@@ -71,8 +74,12 @@ constexpr int kWave = 64;
 // K1 (the SpMV step kernel): one stencil row per lane, kK1 lanes per block
 // (a tuning choice: 64 or 256; larger blocks leave fewer partials for K2).
 constexpr int kRed = 256;         // single-block reductions
-constexpr int kK2 = 256;          // K2: kK2Rows rows per lane
+constexpr int kK2 = 256;          // K2 of the mixed path: kK2Rows rows per lane
 constexpr int kK2Rows = 8;
+constexpr int kGroup = 4;         // K1 partials that K2 adds first
+constexpr int kRunRows = kRed * kGroup;   // rows per block of K2 and k_lz_run of the plain path, one per lane
+constexpr unsigned long long kRunEmpty = ~0ull;  // a partial sum no block has written yet
+constexpr unsigned kRunNoZ = ~0u;                // the same for an entry of z
 constexpr int kBisect = 256;      // shifts per multisection round
 constexpr int kInvitIters = 2;
 constexpr size_t kInvitBytes = 7 * sizeof(double) + 1;  // LDS bytes per row of T in k_tri_vec
@@ -99,6 +106,7 @@ struct LzState {
   double vals[kMaxEig];  // screened Ritz values
   double res[kMaxEig];   // residuals |beta_m s_{m,j}|
   int sel[kMaxEig];      // row of S holding the Ritz vector of vals[j]
+  int stalled;           // 1: a wait of k_lz_run ran out of polls, its steps are void
 };
 
 template <typename T>
@@ -106,6 +114,48 @@ __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v = v + __shfl_xor(v, o, 64);
   return v;
+}
+
+// The same sum of doubles without LDS permutes: lane i adds lane i ^ o for o
+// = 32, 16 (row swaps), 8, 4 (after the earlier steps the values repeat every
+// 2 o lanes, so a rotation by o within 16 lanes reads lane i ^ o's value), 2
+// and 1 (quad permutes).
+template <int CTRL>
+__device__ __forceinline__ double dpp_double(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+template <>
+__device__ __forceinline__ double wave_sum<double>(double v) {
+  {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+  {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+  v = v + dpp_double<0x128>(v);
+  v = v + dpp_double<0x124>(v);
+  v = v + dpp_double<0x4e>(v);
+  v = v + dpp_double<0xb1>(v);
+  return v;
+}
+
+// Sum of red[0..15] for one wave: lane i adds lane i ^ o for o = 8, 4, 2, 1.
+__device__ __forceinline__ double sum16(const double* red) {
+  double v = red[threadIdx.x & 15];
+  v = v + dpp_double<0x128>(v);
+  v = v + dpp_double<0x124>(v);
+  v = v + dpp_double<0x4e>(v);
+  return v + dpp_double<0xb1>(v);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
 // Sum over the block in a fixed order; every thread gets the result.
@@ -214,26 +264,299 @@ __global__ __launch_bounds__(kK1) void k_lz1(LzBufs b, StencilOffsets so, int t)
   if (threadIdx.x == 0) b.part[lb] = s;
 }
 
-__global__ __launch_bounds__(kK2) void k_lz2(LzBufs b, int t) {
-  __shared__ double red[kK2 / kWave];
+__global__ __launch_bounds__(kRunRows) void k_lz2(LzBufs b, int t) {
+  __shared__ double red[kRunRows / kWave];
   const int k = b.st->k + t;
   const float* qk = b.st->V + (size_t)k * b.vstride;
   float* zc = (k & 1) ? b.z1 : b.z0;
-  const float alpha = (float)sum_partials<kK2>(b.part, b.nb1, red);
-  if (blockIdx.x == 0 && threadIdx.x == 0) b.alpha[k] = alpha;
-  double nrm = 0;
-  const int base = blockIdx.x * kK2 * kK2Rows + threadIdx.x;
+  const int row = blockIdx.x * kRunRows + threadIdx.x;
+  // K1's partials: groups of kGroup in order, then sum_partials<kRed> over the
+  // groups, on the first waves
+  double v = 0;
+  if (threadIdx.x < kRed) {
+    for (int i = threadIdx.x * kGroup; i < b.nb1; i += kRed * kGroup) {
+      double g = b.part[i];
 #pragma unroll
-  for (int j = 0; j < kK2Rows; j++) {
-    const int i = base + j * kK2;
-    if (i < b.n) {
-      const float zj = fmaf(-alpha, qk[i], zc[i]);
-      zc[i] = zj;
-      nrm = fma((double)zj, (double)zj, nrm);
+      for (int u = 1; u < kGroup; u++) g += i + u < b.nb1 ? b.part[i + u] : 0.0;
+      v += g;
     }
+    v = wave_sum(v);
+    if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = v;
   }
-  const double s = block_sum<kK2>(nrm, red);
-  if (threadIdx.x == 0) b.part2[blockIdx.x] = s;
+  const float q = row < b.n ? qk[row] : 0.0f, z = row < b.n ? zc[row] : 0.0f;
+  __syncthreads();
+  v = red[0];
+#pragma unroll
+  for (int i = 1; i < kRed / kWave; i++) v += red[i];
+  __syncthreads();
+  const float alpha = (float)v;
+  if (blockIdx.x == 0 && threadIdx.x == 0) b.alpha[k] = alpha;
+  const float zj = fmaf(-alpha, q, z);
+  if (row < b.n) zc[row] = zj;
+  const double s = wave_sum(row < b.n ? (double)zj * (double)zj : 0.0);
+  if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = s;
+  __syncthreads();
+  if (threadIdx.x < kWave) {
+    const double t = sum16(red);
+    if (threadIdx.x == 0) b.part2[blockIdx.x] = t;
+  }
+}
+
+// Rows of the radius-5 disc: |dx| <= half_width(dy), raster order.
+__host__ __device__ constexpr int half_width(int dy) {
+  return dy == 0 ? 5 : (dy >= -3 && dy <= 3) ? 4 : (dy == 4 || dy == -4) ? 3 : 0;
+}
+
+// Values that other blocks of the running grid write or read: accesses at
+// device scope, which go past the per-XCD caches.
+template <typename T>
+__device__ __forceinline__ T shared_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void shared_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// base[off / sizeof(T)] by a byte offset below 4 GiB: a scalar base and one
+// register of address.
+template <typename T>
+__device__ __forceinline__ T* at_byte(T* base, unsigned off) {
+  return (T*)((char*)base + off);
+}
+template <typename T>
+__device__ __forceinline__ const T* at_byte(const T* base, unsigned off) {
+  return (const T*)((const char*)base + off);
+}
+// A copy the compiler knows nothing about: what is computed from it stays in
+// the loop that computes it instead of holding registers across it.
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+// Every memory access this wave issued has completed.
+__device__ __forceinline__ void drain_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Up to N values at byte offsets at[u] of base, each awaited until its block has written it (kEmpty
+// before that): at most `polls` rounds of reads; then, or once another block
+// gave up, st->stalled is set and false returned.  live: bit u set where v[u]
+// is wanted.
+template <int N, typename T>
+__device__ __forceinline__ bool await(const T* base, const unsigned (&at)[N], unsigned live, T kEmpty, LzState* st,
+                                      int polls, T (&v)[N]) {
+  for (int i = 0;; i++) {
+    bool all = true;
+#pragma unroll
+    for (int u = 0; u < N; u++)
+      if (live >> u & 1) v[u] = shared_load(at_byte(base, at[u]));
+#pragma unroll
+    for (int u = 0; u < N; u++)
+      if ((live >> u & 1) && v[u] == kEmpty) all = false;
+    if (all) return true;
+    if (i >= polls || ((i & 63) == 63 && shared_load(&st->stalled))) {
+      shared_store(&st->stalled, 1);
+      return false;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
+__global__ void k_lz_slots(unsigned long long* slots, int count, unsigned* z, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < count) slots[i] = kRunEmpty;
+  if (i < n) z[i] = kRunNoZ;
+}
+
+// `steps` plain steps from step k0 in one launch, bit-identical to
+// k_lz1<256> / k_lz2.  Two kernels per step read the 50 MB matrix (481x321)
+// for every vector and wait for two launches: 16.8 us a step.  Here every
+// block stays resident, so each lane keeps its row's 81 matrix entries, its z
+// and its last q in registers and a step moves the stencil halo of z, the
+// basis row and two partial sums per block: 6.3 us, bound by the two
+// exchanges (about 3,800 cycles each of 15,000) and the 81 LDS reads per row
+// (3,500).
+//  * Rows are consecutive, so halo and sums keep the linear indexing and the
+//    order of the two-kernel step.
+//  * A value that other blocks wait for carries its own flag: slots and z
+//    hold a NaN pattern that no sum or product produces until their block has
+//    written them (an input with that very NaN ends in the stalled path).  So
+//    z needs no fence before the partial that follows it, and the halo is
+//    read while |z|^2 is summed.
+//  * A slot is emptied one exchange after its value was read by all: a block
+//    publishes exchange e + 1 only after it has seen all of e, so whoever has
+//    all of e + 1 knows that e is read everywhere.  Slots alternate between
+//    two sets per sum, z between z0 and z1.  Emptied values have arrived
+//    (drain_memory) before the partial that lets others look at them.
+//  * Reads that come too early delay the stores they wait for: a first look
+//    1,024 cycles after the store takes 3,700 cycles for the sum against
+//    6,500 at once.
+//  * Every wait is bounded; one that runs out sets st->stalled, which ends
+//    all others, and the host runs the solve again with two kernels per step.
+__global__ __launch_bounds__(kRunRows) void k_lz_run(LzBufs b, int w, int halo, int k0, int steps,
+                                                     unsigned long long* slots, int stride, int polls) {
+  extern __shared__ float qs[];  // q of rows [base - halo, base + kRunRows + halo)
+  __shared__ double red[kRunRows / kWave];
+  __shared__ float coef[2];  // alpha; beta
+  __shared__ int quit;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
+  const int base = blockIdx.x * kRunRows, row = base + tid;
+  const bool live = row < b.n;
+  const auto row4 = [&]() { return (unsigned)(base + opaque(tid)) * 4u; };
+  float* V = b.st->V;
+  float a[kStencilArea];
+  const unsigned row0 = row4();
+#pragma unroll
+  for (int d = 0; d < kStencilArea; d++) a[d] = live ? *at_byte(b.A + (size_t)d * b.pitch, row0) : 0.0f;
+  if (tid == 0) quit = 0;
+  __syncthreads();
+  // the halo's z to LDS, as it is
+  auto load_halo = [&](const float* zp) {
+    constexpr int kLoads = 5;
+    for (int i0 = opaque(tid); i0 < 2 * halo; i0 += kLoads * kRunRows) {
+      unsigned at[kLoads], v[kLoads], want = 0;
+#pragma unroll
+      for (int u = 0; u < kLoads; u++) {
+        const int i = i0 + u * kRunRows, c = base - halo + (i < halo ? i : i + kRunRows);
+        const bool in = i < 2 * halo && (unsigned)c < (unsigned)b.n;
+        at[u] = in ? (unsigned)c * 4u : 0u;
+        v[u] = 0;
+        want |= (in ? 1u : 0u) << u;
+      }
+      if (!await<kLoads>((const unsigned*)zp, at, want, kRunNoZ, b.st, polls, v)) {
+        quit = 1;
+        return;
+      }
+#pragma unroll
+      for (int u = 0; u < kLoads; u++) {
+        const int i = i0 + u * kRunRows;
+        if (i < 2 * halo) qs[i < halo ? i : i + kRunRows] = __uint_as_float(v[u]);
+      }
+    }
+  };
+  // wave 0: the sum of an exchange's partials, one per block, in
+  // sum_partials<kRed>'s order
+  auto sum_slots = [&](const unsigned long long* sl) {
+    constexpr int kLoads = kRed / kWave;
+    const int l = opaque(lane);
+    unsigned long long v[kLoads];
+    unsigned at[kLoads], want = 0;
+#pragma unroll
+    for (int u = 0; u < kLoads; u++) {
+      const int i = l + u * kWave;
+      at[u] = i < (int)gridDim.x ? (unsigned)i * 8u : 0u;
+      v[u] = 0;
+      want |= (i < (int)gridDim.x ? 1u : 0u) << u;
+    }
+    if (!await<kLoads>(sl, at, want, kRunEmpty, b.st, polls, v)) quit = 1;
+    double t = wave_sum(__longlong_as_double((long long)v[0]));
+#pragma unroll
+    for (int u = 1; u < kLoads; u++) t += wave_sum(__longlong_as_double((long long)v[u]));
+    return t;
+  };
+  float z = 0, qp = 0;
+  {
+    const float* zp = (k0 & 1) ? b.z0 : b.z1;
+    if (live) z = *at_byte(zp, row4());
+    load_halo(zp);
+    if (k0 > 0) {
+      if (live) qp = *at_byte(V + (size_t)(k0 - 1) * b.vstride, row4());
+      if (wave == 0) {
+        const float beta = (float)sqrt(sum_slots((const unsigned long long*)b.part2));
+        if (lane == 0) coef[1] = beta;
+      }
+    }
+    __syncthreads();
+    if (quit) return;
+  }
+  for (int s = 0; s < steps; s++) {
+    const int k = k0 + s;
+    float* zp = (k & 1) ? b.z0 : b.z1;
+    float* zc = (k & 1) ? b.z1 : b.z0;
+    unsigned long long* sla = slots + (size_t)((s & 1) * 2) * stride;
+    unsigned long long* slb = sla + stride;
+    unsigned long long* sla2 = slots + (size_t)((~s & 1) * 2) * stride;  // the next step's
+    unsigned long long* slb2 = sla2 + stride;
+    float inv = 1, nbeta = 0;
+    if (k > 0) {
+      const float beta = coef[1];
+      if (blockIdx.x == 0 && tid == 0) b.beta[k - 1] = beta;
+      inv = 1.0f / beta;
+      nbeta = -beta;
+    }
+    // every lane scales the halo values it loaded
+    for (int i = opaque(tid); i < 2 * halo; i += kRunRows) {
+      const int o = i < halo ? i : i + kRunRows, c = base - halo + o;
+      qs[o] = (unsigned)c < (unsigned)b.n ? qs[o] * inv : 0.0f;
+    }
+    const float qv = z * inv;
+    qs[halo + tid] = live ? qv : 0.0f;
+    if (live) *at_byte(V + (size_t)k * b.vstride, row4()) = qv;
+    __syncthreads();
+    float acc = 0;
+    {
+      int d = 0;
+#pragma unroll
+      for (int dy = -5; dy <= 5; dy++) {
+        const float* q = qs + halo + tid + dy * w;
+#pragma unroll
+        for (int dx = -half_width(dy); dx <= half_width(dy); dx++) acc = fmaf(a[d++], q[dx], acc);
+      }
+    }
+    if (k > 0) acc = fmaf(nbeta, qp, acc);
+    z = acc;
+    qp = qv;
+    {
+      const double t = wave_sum(live ? (double)qv * (double)z : 0.0);
+      if (lane == 0) red[wave] = t;
+    }
+    drain_memory();  // the emptied slots and z of the last step, before this step's partials
+    __syncthreads();
+    if (wave == 0) {
+      constexpr int kPer = kRed / kWave;
+      double t = red[(lane & (kGroup - 1)) * kPer];
+#pragma unroll
+      for (int i = 1; i < kPer; i++) t += red[(lane & (kGroup - 1)) * kPer + i];
+      double sum = lane_value(t, 0);
+#pragma unroll
+      for (int g = 1; g < kGroup; g++) sum += lane_value(t, g);
+      if (lane == 0) {
+        shared_store(sla + blockIdx.x, (unsigned long long)__double_as_longlong(sum));
+        shared_store(sla2 + blockIdx.x, kRunEmpty);
+      }
+      __builtin_amdgcn_s_sleep(16);  // in units of 64 cycles
+      const float alpha = (float)sum_slots(sla);
+      if (lane == 0) coef[0] = alpha;
+    }
+    __syncthreads();
+    if (quit) return;
+    const float alpha = coef[0];
+    if (blockIdx.x == 0 && tid == 0) b.alpha[k] = alpha;
+    z = fmaf(-alpha, qv, z);
+    if (live) {
+      shared_store(at_byte((unsigned*)zc, row4()), __float_as_uint(z));
+      shared_store(at_byte((unsigned*)zp, row4()), kRunNoZ);
+    }
+    {
+      const double t = wave_sum(live ? (double)z * (double)z : 0.0);
+      if (lane == 0) red[wave] = t;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const double t = sum16(red);
+      if (lane == 0) {
+        shared_store(slb + blockIdx.x, (unsigned long long)__double_as_longlong(t));
+        shared_store(slb2 + blockIdx.x, kRunEmpty);
+        if (s == steps - 1) b.part2[blockIdx.x] = t;
+      }
+    }
+    if (s == steps - 1) return;
+    load_halo(zc);
+    if (wave == 0) {
+      const float beta = (float)sqrt(sum_slots(slb));
+      if (lane == 0) coef[1] = beta;
+    }
+    __syncthreads();
+    if (quit) return;
+  }
 }
 
 // beta of the last step m-1 (needed by the check's residuals).
@@ -963,6 +1286,7 @@ __global__ void k_init(LzState* st, float* V, Z* z1, float q0, int n) {
     st->nscreened = 0;
     st->fail = 0;
     st->m = 0;
+    st->stalled = 0;
   }
   if (i < n) {
     V[i] = q0;
@@ -1082,7 +1406,7 @@ int add_steps(hipGraph_t g, const Steps& p, int steps) {
     } else {
       const void* fn = p.k1 == 64 ? (const void*)&k_lz1<64> : (const void*)&k_lz1<256>;
       DMSC_TRY(add_node(g, &last, fn, dim3(p.plain.nb1), dim3(p.k1 == 64 ? 64 : 256), 0, p.plain, p.so, t));
-      DMSC_TRY(add_node(g, &last, (const void*)&k_lz2, dim3(p.plain.nb2), dim3(kK2), 0, p.plain, t));
+      DMSC_TRY(add_node(g, &last, (const void*)&k_lz2, dim3(p.plain.nb2), dim3(kRunRows), 0, p.plain, t));
     }
   }
   return DMSC_OK;
@@ -1110,6 +1434,64 @@ int run_steps(Ctx* ctx, const Steps& p, LzState* st, int w, int first, int steps
   hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, ctx->stream, st, first);
   DMSC_HIP(hipGetLastError());
   DMSC_HIP(hipGraphLaunch(it->second, ctx->stream));
+  return DMSC_OK;
+}
+
+// Plain solves in progress per device.  k_lz_run needs its whole grid
+// resident; a second one beside it could hold the compute units the first
+// still waits for.  (Kernels that end by themselves only delay it: six images
+// over four batch lanes take 33 ms with it, 38 ms with two kernels per step.)
+class PlainSolve {
+ public:
+  explicit PlainSolve(int device) : device_(device) {
+    std::lock_guard<std::mutex> lk(lock());
+    ++count()[device_];
+  }
+  ~PlainSolve() {
+    std::lock_guard<std::mutex> lk(lock());
+    --count()[device_];
+  }
+  PlainSolve(const PlainSolve&) = delete;
+  PlainSolve& operator=(const PlainSolve&) = delete;
+  bool alone() const {
+    std::lock_guard<std::mutex> lk(lock());
+    return count()[device_] == 1;
+  }
+
+ private:
+  static std::mutex& lock() {
+    static std::mutex m;
+    return m;
+  }
+  static std::map<int, int>& count() {
+    static std::map<int, int> c;
+    return c;
+  }
+  int device_;
+};
+
+size_t run_lds(int halo) { return sizeof(float) * (kRunRows + 2 * (size_t)halo); }
+
+// Whether k_lz_run can take an image of n pixels on this device: every
+// block on a compute unit of its own, its rows and their halo in LDS, and
+// the stencil in the raster order the kernel unrolls.
+int run_fits(int device, int n, const StencilOffsets& so, int w, bool* fits) {
+  *fits = false;
+  const int blocks = div_up(n, kRunRows);
+  constexpr size_t kStatic = 16 * 1024;  // bound of the kernel's own arrays
+  int cus = 0, lds = 0;
+  DMSC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  DMSC_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+  if (blocks > cus || blocks > kRed || run_lds(so.halo) + kStatic > (size_t)lds) return DMSC_OK;
+  int d = 0;
+  for (int dy = -5; dy <= 5; dy++)
+    for (int dx = -half_width(dy); dx <= half_width(dy); dx++, d++)
+      if (d >= kStencilArea || so.off[d] != dy * w + dx) return DMSC_OK;
+  DMSC_HIP(hipFuncSetAttribute((const void*)k_lz_run, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)(lds - kStatic)));
+  int per_cu = 0;
+  DMSC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_lz_run, kRunRows, run_lds(so.halo)));
+  *fits = d == kStencilArea && per_cu >= 1;
   return DMSC_OK;
 }
 
@@ -1182,11 +1564,11 @@ StepShape default_shape(int w, int h, bool mixed) {
 // *ms_per_step (the measurement mode of dmsc_lanczos_time_steps).  `force`
 // selects the step-kernel shape (the autotuner's trials); otherwise the
 // autotuned shape of this size, else the process-wide tuning values.
-// convert == false: A already holds L_sym (a later timing run on the same
+// run == false: never k_lz_run.  convert == false: A already holds L_sym (a later timing run on the same
 // matrix).
 int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool mixed, float* h_eigvals,
           float* d_eigvecs, int* iterations, int time_steps = 0, float* ms_per_step = nullptr,
-          const StepShape* force = nullptr, bool convert = true) {
+          const StepShape* force = nullptr, bool convert = true, bool run = true) {
   const StepShape shape = force ? *force : default_shape(w, h, mixed);
   hipStream_t s = ctx->stream;
   const int n = w * h;
@@ -1232,7 +1614,7 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
     }
   }
   const int nb1 = tile_h ? div_up(w, tile_w) * div_up(h, tile_h) : div_up(n, k1);
-  const int nb2 = div_up(n, kK2 * kK2Rows);
+  const int nb2 = mixed ? div_up(n, kK2 * kK2Rows) : div_up(n, kRunRows);
   int period = mixed ? kGraphSteps : kCheckIter;  // the plain path checks every 500 (lanczos.cu:519)
   const double stop_tol = mixed ? (double)tol * std::pow(10.0, -lanczos_mixed_stop) : (double)tol;
   const int nblk = std::min(div_up(n, 256), 1024);
@@ -1256,6 +1638,8 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
   const int nvrows = mixed ? kMaxCand : kMaxEig;  // rows of S: candidates (mixed) or screened values
   const size_t o_S = carve(sizeof(double) * nvrows * (kMaxIter + 2));
   const size_t o_work = carve(sizeof(double) * 6 * nvrows * (kMaxIter + 2));
+  const int slot_stride = std::max(nb1, nb2);
+  const size_t o_slots = carve(mixed ? 0 : sizeof(unsigned long long) * 4 * slot_stride);
   const size_t o_resall = carve(sizeof(double) * kMaxCand);
   const size_t o_mm = carve(sizeof(float) * 2 * kMaxEig * nblk), o_fin = carve(sizeof(float) * 2 * kMaxEig);
   void* base;
@@ -1366,6 +1750,20 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
     return DMSC_OK;
   }
 
+  // Plain steps in one resident launch per check period where the grid fits
+  // the device (262,144 rows on 256 compute units) and no other plain solve
+  // runs beside this one; 500 steps with their check take 3.3 ms against 5.9
+  // at 61x37, 3.6 against 7.4 at 481x321, 4.7 against 10.2 at 512x512 and,
+  // with the widest halo, 7.5 against 9.5 at 3000x80.
+  std::unique_ptr<PlainSolve> gate;
+  bool resident = false;
+  unsigned long long* slots = (unsigned long long*)(B + o_slots);
+  if (!mixed) {
+    gate = std::make_unique<PlainSolve>(ctx->device);
+    if (k1 == kRed && run && lanczos_run_polls > 0)
+      DMSC_TRY(run_fits(ctx->device, n, p.so, w, &resident));
+  }
+
   int eigCheck = nvec + kCullumExtra;
   int done = 0, prev_m = 0, prev_n = 0;  // prev_n: Ritz values of the last check left in wv
   double prev_res = 0;
@@ -1410,8 +1808,16 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
       cap = ncap;
       hipLaunchKernelGGL(k_set_basis, dim3(1), dim3(1), 0, s, st, V);
     }
-    for (int t = ahead; t < steps; t += kGraphSteps)
-      DMSC_TRY(run_steps(ctx, p, st, w, done + t, std::min(kGraphSteps, steps - t)));
+    if (resident && gate->alone()) {
+      hipLaunchKernelGGL(k_lz_slots, dim3(div_up(std::max(4 * slot_stride, n), 256)), dim3(256), 0, s, slots,
+                         4 * slot_stride, (unsigned*)((done & 1) ? p.plain.z1 : p.plain.z0), n);
+      hipLaunchKernelGGL(k_lz_run, dim3(div_up(n, kRunRows)), dim3(kRunRows), run_lds(p.so.halo), s, p.plain, w,
+                         p.so.halo, done, steps, slots, slot_stride, lanczos_run_polls);
+      DMSC_HIP(hipGetLastError());
+    } else {
+      for (int t = ahead; t < steps; t += kGraphSteps)
+        DMSC_TRY(run_steps(ctx, p, st, w, done + t, std::min(kGraphSteps, steps - t)));
+    }
     done += steps;
     ahead = 0;
     if (mixed) {
@@ -1457,6 +1863,11 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
         DMSC_HIP(hipEventSynchronize(ev_chk));
       } else {
         DMSC_HIP(hipStreamSynchronize(s));
+      }
+      if (hs.stalled) {  // the grid was not resident in time: the same solve with two kernels per step
+        gate.reset();
+        return solve(ctx, w, h, A, pitch, nvec, tol, mixed, h_eigvals, d_eigvecs, iterations, 0, nullptr, force, false,
+                     false);
       }
       if (lanczos_trace) {
         double r = 0;

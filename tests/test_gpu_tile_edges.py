@@ -166,3 +166,31 @@ def test_affinity_windows(ctx, w, h):
     assert np.allclose(host(rs).ravel(), 1 / np.sqrt(d64), rtol=82 * 2.0 ** -24, atol=0)
     L = host(m)[:, :n]
     assert np.allclose(L[40], (d64 - got[40, :n]) / d64, rtol=0, atol=82 * 2.0 ** -24)
+
+
+# plain Lanczos steps in one launch: 1,024 rows per block, partial sums per 256
+# rows; with one poll allowed the launch gives up and two kernels per step run
+@pytest.mark.parametrize("w,h", [(32, 32), (41, 25), (64, 48), (97, 83), (230, 57)])
+def test_resident_lanczos_steps(ctx, w, h):
+    print(f"case: plain Lanczos {w}x{h}", flush=True)
+    y, x = np.mgrid[:h, :w]
+    cell = (x // 13 + 2 * (y // 11)) % 4
+    pb = (0.4 * ((np.diff(cell, axis=1, append=cell[:, -1:]) != 0) | (np.diff(cell, axis=0, append=cell[-1:]) != 0))
+          + 0.02 * np.random.RandomState(w).rand(h, w)).astype(np.float32)
+    out = []
+    for polls in (0, 1 << 16, 1):
+        with dm.tuned(lanczos_run_polls=polls, lanczos_max_iter=1500):
+            try:
+                vals, vecs, it = ctx.generalized_eigensolve(w, h, ctx.intervene(ctx.upload(pb)), nvec=5)
+                out.append((bits(vals), bits(host(vecs)), it))
+            except dm.DmscError as e:
+                out.append(str(e))
+    for got in out[1:]:
+        assert type(got) is type(out[0])
+        if isinstance(got, str):
+            assert got == out[0]
+        else:
+            assert got[2] == out[0][2]
+            np.testing.assert_array_equal(got[0], out[0][0])
+            np.testing.assert_array_equal(got[1], out[0][1])
+    assert not isinstance(out[0], str)
