@@ -234,9 +234,9 @@ int dmsc_tune_set(const char* key, int value) {
     lanczos_k1_threads = value;
     return DMSC_OK;
   }
-  if (!std::strcmp(key, "lanczos_run_polls")) {
-    DMSC_ARG(value >= 0 && value <= 1 << 20, "lanczos_run_polls must be in [0, 2^20]");
-    lanczos_run_polls = value;
+  if (!std::strcmp(key, "resident_polls")) {
+    DMSC_ARG(value >= 0 && value <= 1 << 20, "resident_polls must be in [0, 2^20]");
+    resident_polls = value;
     return DMSC_OK;
   }
   if (!std::strcmp(key, "lanczos_mixed_fused")) {
@@ -339,8 +339,8 @@ int dmsc_tune_get(const char* key, int* value) {
     *value = lanczos_mixed_stop;
     return DMSC_OK;
   }
-  if (!std::strcmp(key, "lanczos_run_polls")) {
-    *value = lanczos_run_polls;
+  if (!std::strcmp(key, "resident_polls")) {
+    *value = resident_polls;
     return DMSC_OK;
   }
   if (!std::strcmp(key, "lanczos_check_max")) {

@@ -10,7 +10,8 @@
 // wanted vectors converge at a rate set by their gap to the 33rd eigenvalue
 // rather than to the 10th, and a filter step has no reduction.  One outer
 // iteration:
-//   1. deg filter steps y = alpha (A x - c x) - beta z, one kernel each
+//   1. deg filter steps y = alpha (A x - c x) - beta z, one kernel each or, on
+//      images of the size where that pays, one kernel for all (k_cheb_run)
 //      (the scaled three-term recurrence, so the block stays O(1)); deg is
 //      50 at first, then whatever cuts the slowest wanted vector's error
 //      tenfold given the current Ritz values (30..300);
@@ -36,6 +37,7 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -43,6 +45,7 @@
 #include "dmsc_device.hpp"
 #include "dmsc_internal.hpp"
 #include "kernels.hpp"
+#include "resident.hpp"
 
 namespace dmsc {
 
@@ -672,6 +675,303 @@ __global__ __launch_bounds__(1024) void k_cheb_gram_sum(int nblk, const double* 
   }
 }
 
+// ---- a whole filter in one launch
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// First of the 81 matrix values of a lane that belong to column offset dx
+// (offsets ascending).  Offset dx has 2 hm + 1 values (hm =
+// half_height(dx)); value k is that of dy = k - hm - i, i the lane's row in
+// its group of four, wrapped into [-hm, hm]: at input row yy = k - hm of the
+// group every row i <= k reads its value k, and the rows that have not
+// reached that input row yet keep in the same place the value they need 2 hm
+// + 1 rows later.  So the four rows' values at one input row sit in one
+// register, without a zero stored for the rows it is no neighbour of.
+__host__ __device__ constexpr int pack_start(int dx) {
+  int at = 0;
+  for (int d = -5; d < dx; d++) at += 2 * half_height(d) + 1;
+  return at;
+}
+
+// One group of rows: per input pixel of the group's columns (position P:
+// column offsets ascending, input rows ascending within one) the lane reads
+// four vectors of one plane from LDS, kAhead positions ahead, and
+// v_mfma_f32_4x4x1_16b_f32 adds 16 outer products (16 columns) of the four
+// rows' matrix values and four vectors, each element one fused multiply-add.
+// The scheduling barriers keep that order of reads and sums: left alone, the
+// compiler reads one position ahead and waits for LDS at every one.
+constexpr int kRunW = 32, kRunSW = kRunW + 10;  // tile width; with its frame
+constexpr int kRunPos = kStencilArea + 3 * 11;
+__host__ __device__ constexpr int pos_dx(int p) {
+  int dx = -5;
+  while (p >= 4 + 2 * half_height(dx)) p -= 4 + 2 * half_height(dx++);
+  return dx;
+}
+__host__ __device__ constexpr int pos_row(int p) {  // input row + half_height
+  int dx = -5;
+  while (p >= 4 + 2 * half_height(dx)) p -= 4 + 2 * half_height(dx++);
+  return p;
+}
+__host__ __device__ constexpr int pos_slot(int p) {
+  return ((pos_row(p) - half_height(pos_dx(p)) + 5) * kRunSW + pos_dx(p)) * 4;
+}
+template <int P, int kAhead>
+__device__ __forceinline__ void run_positions(const float (&a)[kStencilArea], int i, const float4* s0,
+                                              float4 (&b)[kRunPos], f32x4 (&acc)[4]) {
+  if constexpr (P < kRunPos) {
+    constexpr int HM = half_height(pos_dx(P)), K = pos_row(P), AT = pack_start(pos_dx(P)) + K % (2 * HM + 1);
+    // i anew per column, or the masked values of all columns are kept
+    if constexpr (K == 0) asm volatile("" : "+v"(i));
+    if constexpr (P + kAhead < kRunPos) {
+      constexpr int kSlot = pos_slot(P + kAhead);
+      b[P + kAhead] = s0[kSlot];
+    }
+    float av = a[AT];
+    if (K < 3 && HM > 0) av = i <= K ? av : 0.f;
+    if (K > 2 * HM && HM > 0) av = i >= K - 2 * HM ? av : 0.f;
+    if (HM == 0) av = i == K ? av : 0.f;
+    acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, b[P].x, acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, b[P].y, acc[1], 0, 0, 0);
+    acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, b[P].z, acc[2], 0, 0, 0);
+    acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(av, b[P].w, acc[3], 0, 0, 0);
+    if constexpr (P + kAhead < kRunPos) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
+    run_positions<P + 1, kAhead>(a, i, s0, b, acc);
+  }
+}
+template <int P, int kAhead>
+__device__ __forceinline__ void first_reads(const float4* s0, float4 (&b)[kRunPos]) {
+  if constexpr (P < kAhead) {
+    constexpr int kSlot = pos_slot(P);
+    b[P] = s0[kSlot];
+    first_reads<P + 1, kAhead>(s0, b);
+  }
+}
+template <int kAhead>
+__device__ __forceinline__ void run_unit(const float (&a)[kStencilArea], int i, const float4* s0, f32x4 (&acc)[4]) {
+  float4 b[kRunPos];
+  first_reads<0, kAhead>(s0, b);
+  __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+  run_positions<0, kAhead>(a, i, s0, b, acc);
+}
+
+// Coefficients of a filter: step k is y = alpha[k] (A x - c x) - beta[k] z.
+struct RunCoefs {
+  float c;
+  float alpha[kMaxDeg], beta[kMaxDeg];
+};
+
+__global__ void k_cheb_empty(uint4* ring, size_t count, int* stalled) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *stalled = 0;
+  if (i < count) ring[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+}
+
+// Pairs of 16-byte entries at device scope (past the per-XCD caches) through
+// a buffer descriptor: an offset past its range reads 0 and drops a store.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kDeviceScope = 16;  // the sc1 bit of a buffer access
+constexpr int kVolatile = (int)0x80000000;
+constexpr unsigned kNowhere = 0x80000000u;
+constexpr unsigned kRunNone = ~0u;  // an entry no block has written yet
+
+// `deg` filter steps from x0; the last step's block goes to ring (deg % 3).
+// One launch per step reads the matrix four times through L2 and once from
+// memory and stages the block anew: 25.5 us at 481x321, of which 22 are its
+// memory accesses.  Here every block stays resident with its pixels' matrix
+// rows in registers (81 values for each of a lane's pixels: lane 4 b + i of a
+// wave holds row i of column b of a 16 x 4 pixel unit) and a step moves only
+// the frame of its tile: 19.8 us, bound by the reads of the frames and units
+// from LDS (2.8 MB a step and block, 21,900 cycles at 128 bytes each) beside
+// 2,736 matrix instructions per SIMD (25,700 cycles at the rate a plain loop of
+// them reaches), and by the staging between them.
+//  * The 32 vectors go through LDS in two halves of 16 (a 42 x 34 frame takes
+//    91 KB); what a lane holds of the half that is not in LDS stays in
+//    registers.  A half's frame was published half a step before it is needed,
+//    so no wait is in sight of it.
+//  * Only pixels within another tile's reach go to memory, each as its own
+//    flag: all ones (a NaN no sum produces) until written.  There are three
+//    blocks in turn: the entries of the step after next are emptied once this
+//    step's frame is complete (every block this one reads from has then
+//    written the step after the one they held, so nobody reads them), and they
+//    have arrived (drain_memory) before this step's values let others get to
+//    the next.  Reach is symmetric, also where linear indexing couples the
+//    ends of image rows.
+//  * The sums run in the order of the tiles above, matrix entries outside the
+//    disc as 0: bit-identical to one launch per step.
+//  * Waits are bounded; one that runs out sets *stalled, which ends all others,
+//    and the host repeats the filter with one launch per step.
+template <int U>
+__global__ __launch_bounds__(64 * U, U > 8 ? 3 : 2) void k_cheb_run(int w, int h, int ntx, const float* __restrict__ A, size_t pitch,
+                                                     const float4* __restrict__ x0, float4* ring, size_t vs,
+                                                     RunCoefs co, int deg, int* stalled, int polls) {
+  constexpr int TH = 2 * U, SH = TH + 10, NT = 64 * U, kCells = SH * kRunSW;
+  constexpr int kFrame = kCells - kRunW * TH;
+  constexpr int kItems = (kFrame * 4 + NT - 1) / NT;
+  constexpr bool kEarly = U <= 8;  // registers to load the next frame while this one is used
+  constexpr bool kLdsZ = U > 8;   // the registers do not hold both halves' z
+  constexpr int kAhead = U > 8 ? 4 : 6;
+  extern __shared__ float4 sx[];  // [kCells][4 planes], then z of half 0 ([4][NT]) with kLdsZ
+  float4* const sz = sx + kCells * 4;
+  __shared__ unsigned list[kFrame][2];  // frame: cell, byte offset of the pixel it holds in a plane
+  __shared__ int diag[4][kStencilArea];
+  __shared__ int count, quit;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane & 3;
+  const int n = w * h;
+  const int bx = (int)(blockIdx.x % ntx) * kRunW, by = (int)(blockIdx.x / ntx) * TH;
+  const int ex = min(bx + kRunW, w), ey = min(by + TH, h);  // the tile's pixels end here
+  const int lx = (wave & 1) * 16 + (lane >> 2), ly = (wave >> 1) * 4;
+  const int px = bx + lx;
+  if (tid == 0) count = quit = 0;
+  __syncthreads();
+  for (int c = tid; c < kCells; c += NT) {
+    const int gy = by - 5 + c / kRunSW, gx = bx - 5 + c % kRunSW;
+    const bool own = gx >= bx && gx < ex && gy >= by && gy < ey;
+    const int q = gy * w + gx;
+    if (!own && gx < ex + 5 && gy < ey + 5 && (unsigned)q < (unsigned)n) {
+      const int at = atomicAdd(&count, 1);
+      list[at][0] = (unsigned)c;
+      list[at][1] = (unsigned)q * 16u;
+    } else if (!own) {
+      for (int p = 0; p < 4; p++) sx[c * 4 + p] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  }
+  for (int e = tid; e < 4 * kStencilArea; e += NT) {
+    const int i = e / kStencilArea, v = e % kStencilArea;
+    int dx = -5;
+    while (dx < 5 && v >= pack_start(dx + 1)) dx++;
+    const int hm = half_height(dx);
+    int dy = v - pack_start(dx) - hm - i;
+    while (dy < -hm) dy += 2 * hm + 1;
+    diag[i][v] = disc_index(dy, dx);
+  }
+  __syncthreads();
+  const int frame = count;  // at least 1: cell (-1, 0) or (-1, 1) of a tile lies in an image of 2 pixels or more
+  float a[kStencilArea];
+  {
+    const bool live = px < w && by + ly + j < h;
+    const size_t p = live ? (size_t)(by + ly + j) * w + px : 0;
+#pragma unroll
+    for (int v = 0; v < kStencilArea; v++) {
+      const float t = A[(size_t)diag[j][v] * pitch + p];
+      a[v] = live ? t : 0.f;
+    }
+  }
+  const unsigned plane = (unsigned)vs * 16u, row_bytes = (unsigned)w * 16u;
+  const unsigned block_bytes = plane * kPlanes;
+  const unsigned own0 = (unsigned)j * plane + (unsigned)((by + ly) * w + px) * 16u;  // row ly of the lane's plane
+  unsigned mine = 0;  // bits 0-3: rows inside the image; 4-7: within another block's reach
+  float4 held[2][4], z[2][4];  // the halves' current and previous block: rows ly .. ly + 3 of plane j
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int y = by + ly + r;
+    const bool in = px < w && y < h;
+    if (in) mine |= 1u << r;
+    if (in && (px < bx + 5 || px >= ex - 5 || y < by + 5 || y >= ey - 5)) mine |= 16u << r;
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++) {
+      const float4 t = x0[(size_t)(4 * hf + j) * vs + (in ? (size_t)y * w + px : 0)];
+      held[hf][r] = in ? t : make_float4(0.f, 0.f, 0.f, 0.f);
+      z[hf][r] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (kLdsZ && hf == 0) sz[r * NT + tid] = z[hf][r];
+    }
+  }
+  float4* s0 = sx + (ly * kRunSW + lx + 5) * 4 + j;
+
+  const auto block = [&](int b) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(ring + (size_t)(b % 3) * kPlanes * vs), 0, block_bytes, 0x00020000);
+  };
+  // The frame of half hf at step k: x0's in the first step, else what the other
+  // blocks wrote.  Lanes beyond the list repeat its last entry.
+  struct Frame {
+    u32x4 v[kItems];
+  } early;
+  const auto frame_entry = [&](int u) {
+    return min((resident::opaque(tid) >> 2) + u * (NT / 4), frame - 1);
+  };
+  const auto load_frame = [&](u32x4 (&v)[kItems], int hf, int k) {
+    const auto src = k == 0 ? __builtin_amdgcn_make_buffer_rsrc((void*)x0, 0, block_bytes, 0x00020000) : block(k);
+#pragma unroll
+    for (int u = 0; u < kItems; u++)
+      v[u] = __builtin_amdgcn_raw_buffer_load_b128(src, list[frame_entry(u)][1] + (unsigned)j * plane, hf * 4 * plane,
+                                                   kDeviceScope | kVolatile);
+  };
+  const auto await_frame = [&](u32x4 (&v)[kItems], int hf, int k) {
+    for (int i = 0;; i++) {
+      bool all = true;
+#pragma unroll
+      for (int u = 0; u < kItems; u++) all = all && max(max(v[u].x, v[u].y), max(v[u].z, v[u].w)) != kRunNone;
+      if (all) break;
+      if (i >= polls || ((i & 63) == 63 && resident::shared_load(stalled))) {
+        resident::shared_store(stalled, 1);
+        quit = 1;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      load_frame(v, hf, k);
+    }
+  };
+  if (kEarly) load_frame(early.v, 0, 0);
+
+  const auto half = [&](auto HF, int k) {
+    constexpr int hf = decltype(HF)::value;
+    const bool last = k == deg - 1;
+    const auto out = block(k + 1), next = block(k + 2);
+    const unsigned soff = hf * 4 * plane;
+    Frame late;
+    u32x4(&v)[kItems] = kEarly ? early.v : late.v;
+    if (kEarly) await_frame(v, hf, k);
+    __syncthreads();  // the last half's reads are over
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (mine >> r & 1) s0[(r + 5) * kRunSW * 4] = held[hf][r];
+    if (!kEarly) {
+      load_frame(v, hf, k);
+      await_frame(v, hf, k);
+    }
+#pragma unroll
+      for (int u = 0; u < kItems; u++) ((u32x4*)sx)[list[frame_entry(u)][0] * 4 + j] = v[u];
+    __syncthreads();
+    if (quit) return false;
+    // the next step's entries still hold those of three steps before; all have
+    // read them, for every block this one reads from has written the step after
+    if (!last) {
+      const u32x4 none = {kRunNone, kRunNone, kRunNone, kRunNone};
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        __builtin_amdgcn_raw_buffer_store_b128(none, next, (mine >> (4 + r) & 1) ? own0 + r * row_bytes : kNowhere, soff,
+                                               kDeviceScope);
+    }
+    if (kEarly && (!hf || !last)) load_frame(early.v, hf ^ 1, hf ? k + 1 : k);  // the next half's
+    f32x4 acc[4] = {};
+    run_unit<kAhead>(a, resident::opaque(j), s0, acc);
+    const float alpha = co.alpha[k], beta = co.beta[k];
+    resident::drain_memory();  // the emptied entries, before what lets others look at them
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const float4 xo = s0[(r + 5) * kRunSW * 4];
+      const float4 zo = kLdsZ && hf == 0 ? sz[r * NT + tid] : z[hf][r];
+      float4 o;
+      o.x = alpha * mad(-co.c, xo.x, acc[0][r]) - beta * zo.x;
+      o.y = alpha * mad(-co.c, xo.y, acc[1][r]) - beta * zo.y;
+      o.z = alpha * mad(-co.c, xo.z, acc[2][r]) - beta * zo.z;
+      o.w = alpha * mad(-co.c, xo.w, acc[3][r]) - beta * zo.w;
+      if (kLdsZ && hf == 0)
+        sz[r * NT + tid] = xo;
+      else
+        z[hf][r] = xo;
+      held[hf][r] = o;
+      const bool store = (last ? mine >> r : mine >> (4 + r)) & 1;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), out,
+                                             store ? own0 + r * row_bytes : kNowhere, soff, kDeviceScope);
+    }
+    return true;
+  };
+  for (int k = 0; k < deg; k++) {
+    if (!half(std::integral_constant<int, 0>{}, k)) return;
+    if (!half(std::integral_constant<int, 1>{}, k)) return;
+  }
+}
+
 template <int R, int VP, bool F64 = false>
 int launch_step(hipStream_t s, int w, int h, const float* A, size_t pitch, const float4* x,
                 const float4* z, float4* y, size_t vs, double alpha, double c, double beta) {
@@ -819,6 +1119,56 @@ bool chebyshev_shape_valid(int v) {
          v == 2337;
 }
 
+namespace {
+// k_cheb_run's launch for this image: units (of 4 x 16 pixels) per block, 0
+// for one launch per step.  Per product of a whole solve, with one launch per
+// step against k_cheb_run: 28.9 against 25.7 us at 481x321 (12 units), 31.0
+// against 25.3 at 512x384 (12), 26.7 against 20.2 at 400x300 (8), 21.8
+// against 20.0 at 320x240 (8).  Images that fit the device in tiles of 4 units
+// (65,536 pixels on 256 compute units) keep one launch per step: there a step
+// is one chain of dependent sums per SIMD, 14.0 against 14.7 us at 160x120.
+struct RunShape {
+  int units = 0, ntx = 0, blocks = 0;
+  size_t lds = 0;
+};
+template <int U>
+int run_shape_of(int device, int cus, int w, int h, RunShape* rs) {
+  const int ntx = div_up(w, kRunW), blocks = ntx * div_up(h, 2 * U);
+  if (rs->units || blocks > cus) return DMSC_OK;
+  const size_t lds = ((size_t)(2 * U + 10) * kRunSW * 4 + (U > 8 ? 4 * 64 * U : 0)) * sizeof(float4);
+  int lds_max = 0, per_cu = 0;
+  DMSC_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+  if (lds + 8 * 1024 > (size_t)lds_max) return DMSC_OK;
+  DMSC_HIP(hipFuncSetAttribute((const void*)k_cheb_run<U>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  DMSC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_cheb_run<U>, 64 * U, lds));
+  if (per_cu >= 1) *rs = RunShape{U, ntx, blocks, lds};
+  return DMSC_OK;
+}
+int run_shape(int device, int w, int h, RunShape* rs) {
+  int cus = 0;
+  DMSC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  if (div_up(w, kRunW) * div_up(h, 8) <= cus) return DMSC_OK;
+  DMSC_TRY(run_shape_of<8>(device, cus, w, h, rs));
+  DMSC_TRY(run_shape_of<12>(device, cus, w, h, rs));
+  return DMSC_OK;
+}
+
+int launch_run(const RunShape& rs, hipStream_t s, int w, int h, const float* A, size_t pitch, const float4* x0,
+               float4* ring, size_t vs, const RunCoefs& co, int deg, int* stalled) {
+  const size_t count = (size_t)3 * kPlanes * vs;
+  hipLaunchKernelGGL(k_cheb_empty, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, (uint4*)ring, count,
+                     stalled);
+#define RUN_CASE(U)                                                                                               \
+  if (rs.units == U)                                                                                              \
+    hipLaunchKernelGGL(k_cheb_run<U>, dim3(rs.blocks), dim3(64 * U), rs.lds, s, w, h, rs.ntx, A, pitch, x0, ring, \
+                       vs, co, deg, stalled, resident_polls);
+  RUN_CASE(8) RUN_CASE(12)
+#undef RUN_CASE
+  DMSC_HIP(hipGetLastError());
+  return DMSC_OK;
+}
+}  // namespace
+
 // The nvec smallest eigenpairs of L_sym (A, already converted): unit
 // eigenvectors to d_out[j * n + p], eigenvalues to vals; *products = the
 // number of block products with A.
@@ -833,7 +1183,7 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
   const size_t blk = (size_t)kPlanes * vs * sizeof(float4);
   const int nrb = div_up(n, 256);  // k_cheb_resid_rotate blocks
   const size_t o_part = 4 * blk, o_gram = o_part + (size_t)kGrams * nblk * kB * kB * sizeof(double),
-               o_rot = o_gram + (size_t)kGrams * kB * kB * sizeof(double),
+               o_rot = o_gram + ((size_t)kGrams * kB * kB + 2) * sizeof(double),  // with the launch's stall flag
                o_theta = o_rot + (size_t)kB * kB * sizeof(double),
                o_res = o_theta + (size_t)kResidMax * sizeof(double),
                o_rpart = o_res + (size_t)kResidMax * sizeof(double),
@@ -875,32 +1225,58 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
   double cut = kFirstCut;
   int deg = chebyshev_first_degree, total = 0, flat = 0;
   double best = HUGE_VAL;
+  RunShape rs;
+  if (resident_polls > 0 && chebyshev_shape == 0) DMSC_TRY(run_shape(ctx->device, w, h, &rs));
+  std::unique_ptr<ResidentGrid> gate;
+  if (rs.units) gate = std::make_unique<ResidentGrid>(ctx->device);
+  bool whole = gate && gate->held();
+  int* stalled = (int*)(gram + (size_t)kGrams * kB * kB);
+  const int* h_stalled = (const int*)(h_gram + (size_t)kGrams * kB * kB);
+  RunCoefs co;
   for (int outer = 0; outer < kMaxOuter; outer++) {
     // scaled Chebyshev filter of degree deg damping [cut, kUpper], normalised at 0
     const double e = (kUpper - cut) / 2, c = (kUpper + cut) / 2;
     double sigma = e / (0.0 - c);
     const double tau = 2 / sigma;
-    DMSC_TRY(step(shape, s, w, h, A, pitchz, X0, nullptr, ring[0], vs, sigma / e, c, 0.0));
     int cur = 0;
-    const float4* prev = X0;
-    for (int i = 2; i <= deg; i++) {
-      const double sn = 1 / (tau - sigma);
-      const int nx = (cur + 1) % 3;
-      DMSC_TRY(step(shape, s, w, h, A, pitchz, ring[cur], prev, ring[nx], vs, 2 * sn / e, c, sigma * sn));
-      prev = ring[cur];
-      cur = nx;
-      sigma = sn;
+    if (whole) {
+      co.c = (float)c;
+      for (int i = 0; i < deg; i++) {
+        const double sn = 1 / (tau - sigma);
+        co.alpha[i] = (float)(i ? 2 * sn / e : sigma / e);
+        co.beta[i] = (float)(i ? sigma * sn : 0.0);
+        if (i) sigma = sn;
+      }
+      DMSC_TRY(launch_run(rs, s, w, h, A, pitchz, X0, ring[0], vs, co, deg, stalled));
+      cur = deg % 3;
+    } else {
+      DMSC_TRY(step(shape, s, w, h, A, pitchz, X0, nullptr, ring[0], vs, sigma / e, c, 0.0));
+      const float4* prev = X0;
+      for (int i = 2; i <= deg; i++) {
+        const double sn = 1 / (tau - sigma);
+        const int nx = (cur + 1) % 3;
+        DMSC_TRY(step(shape, s, w, h, A, pitchz, ring[cur], prev, ring[nx], vs, 2 * sn / e, c, sigma * sn));
+        prev = ring[cur];
+        cur = nx;
+        sigma = sn;
+      }
     }
     float4* Y = ring[cur];
     float4* Wb = ring[(cur + 1) % 3];
     DMSC_TRY(product_f64(shape, s, w, h, A, pitchz, Y, Wb, vs));
     hipLaunchKernelGGL(k_cheb_gram, dim3(nblk), dim3(256), 0, s, n, vs, chunk, Y, Wb, X0, part);
     hipLaunchKernelGGL(k_cheb_gram_sum, dim3(div_up(kGrams * kB * kB, 64)), dim3(1024), 0, s, nblk, part, gram);
-    DMSC_HIP(hipMemcpyAsync(h_gram, gram, kGrams * kB * kB * sizeof(double), hipMemcpyDeviceToHost, s));
+    DMSC_HIP(hipMemcpyAsync(h_gram, gram, kGrams * kB * kB * sizeof(double) + sizeof(int), hipMemcpyDeviceToHost, s));
     // one host round trip per outer iteration: the Gram matrices of this
     // block and the residuals of the previous Ritz pairs (enqueued last
     // iteration, read here)
     DMSC_HIP(hipStreamSynchronize(s));
+    if (whole && *h_stalled) {  // the grid was not resident in time: this iteration again, one launch per step
+      whole = false;
+      gate.reset();
+      outer--;
+      continue;
+    }
     const auto t_rr = std::chrono::steady_clock::now();
     if (!rayleigh_ritz(h_gram, h_gram + kB * kB, kB, theta, S))
       return fail(DMSC_ERR_INTERNAL, "block eigensolver: filtered block lost rank at outer iteration %d", outer);

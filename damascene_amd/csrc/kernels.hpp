@@ -107,7 +107,7 @@ extern int lanczos_k1_threads;
 // Plain steps in one resident launch per check: most rounds of reads of an
 // awaited value before the launch is given up for two kernels per step (0 =
 // always two kernels).
-extern int lanczos_run_polls;
+extern int resident_polls;
 // Mixed eigensolver step: 2 = one fused kernel per step over pixel tiles
 // (default), 1 = one fused kernel over runs of consecutive rows (when
 // the stencil halo fits in LDS), 0 = two kernels per step.

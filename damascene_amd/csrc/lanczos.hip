@@ -50,6 +50,7 @@
 #include "dmsc_device.hpp"
 #include "dmsc_internal.hpp"
 #include "kernels.hpp"
+#include "resident.hpp"
 #include "tridiag.hpp"
 
 namespace dmsc {
@@ -62,7 +63,7 @@ int lanczos_max_iter = kMaxIter;
 int lanczos_check_max = 0;
 int lanczos_mixed_stop = 4;
 int lanczos_step_loads = 0;
-int lanczos_run_polls = 1 << 14;
+int resident_polls = 1 << 14;
 
 namespace {
 
@@ -307,58 +308,7 @@ __host__ __device__ constexpr int half_width(int dy) {
   return dy == 0 ? 5 : (dy >= -3 && dy <= 3) ? 4 : (dy == 4 || dy == -4) ? 3 : 0;
 }
 
-// Values that other blocks of the running grid write or read: accesses at
-// device scope, which go past the per-XCD caches.
-template <typename T>
-__device__ __forceinline__ T shared_load(const T* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void shared_store(T* p, T v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// base[off / sizeof(T)] by a byte offset below 4 GiB: a scalar base and one
-// register of address.
-template <typename T>
-__device__ __forceinline__ T* at_byte(T* base, unsigned off) {
-  return (T*)((char*)base + off);
-}
-template <typename T>
-__device__ __forceinline__ const T* at_byte(const T* base, unsigned off) {
-  return (const T*)((const char*)base + off);
-}
-// A copy the compiler knows nothing about: what is computed from it stays in
-// the loop that computes it instead of holding registers across it.
-__device__ __forceinline__ int opaque(int v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-// Every memory access this wave issued has completed.
-__device__ __forceinline__ void drain_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// Up to N values at byte offsets at[u] of base, each awaited until its block has written it (kEmpty
-// before that): at most `polls` rounds of reads; then, or once another block
-// gave up, st->stalled is set and false returned.  live: bit u set where v[u]
-// is wanted.
-template <int N, typename T>
-__device__ __forceinline__ bool await(const T* base, const unsigned (&at)[N], unsigned live, T kEmpty, LzState* st,
-                                      int polls, T (&v)[N]) {
-  for (int i = 0;; i++) {
-    bool all = true;
-#pragma unroll
-    for (int u = 0; u < N; u++)
-      if (live >> u & 1) v[u] = shared_load(at_byte(base, at[u]));
-#pragma unroll
-    for (int u = 0; u < N; u++)
-      if ((live >> u & 1) && v[u] == kEmpty) all = false;
-    if (all) return true;
-    if (i >= polls || ((i & 63) == 63 && shared_load(&st->stalled))) {
-      shared_store(&st->stalled, 1);
-      return false;
-    }
-    __builtin_amdgcn_s_sleep(1);
-  }
-}
+using namespace resident;
 
 __global__ void k_lz_slots(unsigned long long* slots, int count, unsigned* z, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -421,7 +371,7 @@ __global__ __launch_bounds__(kRunRows) void k_lz_run(LzBufs b, int w, int halo, 
         v[u] = 0;
         want |= (in ? 1u : 0u) << u;
       }
-      if (!await<kLoads>((const unsigned*)zp, at, want, kRunNoZ, b.st, polls, v)) {
+      if (!await<kLoads>((const unsigned*)zp, at, want, kRunNoZ, &b.st->stalled, polls, v)) {
         quit = 1;
         return;
       }
@@ -446,7 +396,7 @@ __global__ __launch_bounds__(kRunRows) void k_lz_run(LzBufs b, int w, int halo, 
       v[u] = 0;
       want |= (i < (int)gridDim.x ? 1u : 0u) << u;
     }
-    if (!await<kLoads>(sl, at, want, kRunEmpty, b.st, polls, v)) quit = 1;
+    if (!await<kLoads>(sl, at, want, kRunEmpty, &b.st->stalled, polls, v)) quit = 1;
     double t = wave_sum(__longlong_as_double((long long)v[0]));
 #pragma unroll
     for (int u = 1; u < kLoads; u++) t += wave_sum(__longlong_as_double((long long)v[u]));
@@ -1437,39 +1387,6 @@ int run_steps(Ctx* ctx, const Steps& p, LzState* st, int w, int first, int steps
   return DMSC_OK;
 }
 
-// Plain solves in progress per device.  k_lz_run needs its whole grid
-// resident; a second one beside it could hold the compute units the first
-// still waits for.  (Kernels that end by themselves only delay it: six images
-// over four batch lanes take 33 ms with it, 38 ms with two kernels per step.)
-class PlainSolve {
- public:
-  explicit PlainSolve(int device) : device_(device) {
-    std::lock_guard<std::mutex> lk(lock());
-    ++count()[device_];
-  }
-  ~PlainSolve() {
-    std::lock_guard<std::mutex> lk(lock());
-    --count()[device_];
-  }
-  PlainSolve(const PlainSolve&) = delete;
-  PlainSolve& operator=(const PlainSolve&) = delete;
-  bool alone() const {
-    std::lock_guard<std::mutex> lk(lock());
-    return count()[device_] == 1;
-  }
-
- private:
-  static std::mutex& lock() {
-    static std::mutex m;
-    return m;
-  }
-  static std::map<int, int>& count() {
-    static std::map<int, int> c;
-    return c;
-  }
-  int device_;
-};
-
 size_t run_lds(int halo) { return sizeof(float) * (kRunRows + 2 * (size_t)halo); }
 
 // Whether k_lz_run can take an image of n pixels on this device: every
@@ -1751,17 +1668,19 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
   }
 
   // Plain steps in one resident launch per check period where the grid fits
-  // the device (262,144 rows on 256 compute units) and no other plain solve
-  // runs beside this one; 500 steps with their check take 3.3 ms against 5.9
+  // the device (262,144 rows on 256 compute units) and no other resident
+  // launch runs on it; 500 steps with their check take 3.3 ms against 5.9
   // at 61x37, 3.6 against 7.4 at 481x321, 4.7 against 10.2 at 512x512 and,
   // with the widest halo, 7.5 against 9.5 at 3000x80.
-  std::unique_ptr<PlainSolve> gate;
+  // Beside other kernels it holds its own: six images over four batch lanes
+  // take 33 ms with it, 38 ms with two kernels per step.
+  std::unique_ptr<ResidentGrid> gate;
   bool resident = false;
   unsigned long long* slots = (unsigned long long*)(B + o_slots);
   if (!mixed) {
-    gate = std::make_unique<PlainSolve>(ctx->device);
-    if (k1 == kRed && run && lanczos_run_polls > 0)
-      DMSC_TRY(run_fits(ctx->device, n, p.so, w, &resident));
+    if (k1 == kRed && run && resident_polls > 0) DMSC_TRY(run_fits(ctx->device, n, p.so, w, &resident));
+    if (resident) gate = std::make_unique<ResidentGrid>(ctx->device);
+    resident = resident && gate->held();
   }
 
   int eigCheck = nvec + kCullumExtra;
@@ -1808,11 +1727,11 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
       cap = ncap;
       hipLaunchKernelGGL(k_set_basis, dim3(1), dim3(1), 0, s, st, V);
     }
-    if (resident && gate->alone()) {
+    if (resident) {
       hipLaunchKernelGGL(k_lz_slots, dim3(div_up(std::max(4 * slot_stride, n), 256)), dim3(256), 0, s, slots,
                          4 * slot_stride, (unsigned*)((done & 1) ? p.plain.z1 : p.plain.z0), n);
       hipLaunchKernelGGL(k_lz_run, dim3(div_up(n, kRunRows)), dim3(kRunRows), run_lds(p.so.halo), s, p.plain, w,
-                         p.so.halo, done, steps, slots, slot_stride, lanczos_run_polls);
+                         p.so.halo, done, steps, slots, slot_stride, resident_polls);
       DMSC_HIP(hipGetLastError());
     } else {
       for (int t = ahead; t < steps; t += kGraphSteps)

@@ -237,7 +237,7 @@ int dmsc_write_pgm(const char* path, int w, int h, const float* h_data);
  *                         kernel: 0 = automatic (default: 256 for two-kernel
  *                         steps, 512 for the fused mixed step), 64, 256 or
  *                         512 (512 applies to the fused step only).
- *   "lanczos_run_polls":  plain eigensolver: how often a block of the launch
+ *   "resident_polls":  plain eigensolver: how often a block of the launch
  *                         that runs a whole check period looks for another
  *                         block's value before the solve starts over with
  *                         two kernels per step (0-2^20, 16384; 0 = always

@@ -179,7 +179,7 @@ def test_resident_lanczos_steps(ctx, w, h):
           + 0.02 * np.random.RandomState(w).rand(h, w)).astype(np.float32)
     out = []
     for polls in (0, 1 << 16, 1):
-        with dm.tuned(lanczos_run_polls=polls, lanczos_max_iter=1500):
+        with dm.tuned(resident_polls=polls, lanczos_max_iter=1500):
             try:
                 vals, vecs, it = ctx.generalized_eigensolve(w, h, ctx.intervene(ctx.upload(pb)), nvec=5)
                 out.append((bits(vals), bits(host(vecs)), it))
@@ -194,3 +194,32 @@ def test_resident_lanczos_steps(ctx, w, h):
             np.testing.assert_array_equal(got[0], out[0][0])
             np.testing.assert_array_equal(got[1], out[0][1])
     assert not isinstance(out[0], str)
+
+
+# block filter in one launch: tiles of 32 x 16 and 32 x 24 pixels by image size,
+# matrices that couple the ends of image rows, and the restart after a stall
+@pytest.mark.parametrize("w,h", [(31, 2100), (40, 1031), (1025, 64), (261, 257), (330, 390), (500, 375)])
+def test_resident_block_filter(ctx, w, h):
+    print(f"case: block filter {w}x{h}", flush=True)
+    r = np.random.RandomState(w)
+    n = w * h
+    y, x = np.mgrid[:h, :w]
+    cell = ((3 * x // w) + 3 * (2 * y // h)).ravel()
+    m = np.zeros((81, dm.pitch_in_floats(n)), np.float32)
+    for k, (dy, dx) in enumerate((y, x) for y in range(-5, 6) for x in range(-5, 6) if y * y + x * x <= 25):
+        off = dy * w + dx
+        if off >= 0:
+            v = np.zeros(n, np.float32)
+            v[:n - off] = np.where(cell[:n - off] == cell[off:], 1.0, 0.02) * (0.9 + 0.1 * r.rand(n - off))
+            m[k, :n] = v
+            m[80 - k, off:n] = v[:n - off]
+    out = []
+    for polls in (0, 1 << 14, 1):
+        with dm.tuned(resident_polls=polls):
+            vals, vecs, products = ctx.generalized_eigensolve(w, h, ctx.upload(m), nvec=4, tol=1e-2,
+                                                              precision=dm.PREC_MIXED)
+            out.append((bits(vals), bits(host(vecs)), products))
+    for got in out[1:]:
+        assert got[2] == out[0][2]
+        np.testing.assert_array_equal(got[0], out[0][0])
+        np.testing.assert_array_equal(got[1], out[0][1])
