@@ -138,6 +138,10 @@ int dmsc_ctx_create(dmsc_ctx** out, int device, void* stream) {
   // want a private stream create one and pass it in
   c->stream = (hipStream_t)stream;
   c->own_stream = false;
+  if (const int rc = init_walks(c); rc != DMSC_OK) {
+    delete c;
+    return rc;
+  }
   *out = c;
   return DMSC_OK;
 }

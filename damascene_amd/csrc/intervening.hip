@@ -147,24 +147,22 @@ __global__ __launch_bounds__(256) void k_affinities(int w, int h, float rs, cons
   }
 }
 
-// The context's device copy of the walk codes, uploaded once.
-int walk_device(Ctx* ctx, bool narrow, const uint8_t** out) {
-  uint8_t*& d = ctx->d_walks[narrow];
-  if (!d) {
-    const std::vector<uint8_t>& c = walk_codes(narrow);
+}  // namespace
+
+// A context's device copies of the walk codes, uploaded when it is made: the
+// launch itself allocates and copies nothing, so a caller may capture it.
+int init_walks(Ctx* ctx) {
+  for (int narrow = 0; narrow < 2; narrow++) {
+    const std::vector<uint8_t>& c = walk_codes(narrow != 0);
     if (c.empty()) return fail(DMSC_ERR_INTERNAL, "a clipped window crosses an unexpected set of pixels");
-    DMSC_HIP(hipMalloc(&d, c.size()));
-    DMSC_HIP(hipMemcpy(d, c.data(), c.size(), hipMemcpyHostToDevice));
+    DMSC_HIP(hipMalloc(&ctx->d_walks[narrow], c.size()));
+    DMSC_HIP(hipMemcpy(ctx->d_walks[narrow], c.data(), c.size(), hipMemcpyHostToDevice));
   }
-  *out = d;
   return DMSC_OK;
 }
 
-}  // namespace
-
 int launch_intervene(Ctx* ctx, int w, int h, const float* mpb, float* M, int pitch, float sigma) {
-  const uint8_t* T;
-  DMSC_TRY(walk_device(ctx, w < 11 || h < 11, &T));
+  const uint8_t* T = ctx->d_walks[w < 11 || h < 11];
   hipLaunchKernelGGL(k_affinities, dim3(div_up(w, ITX), div_up(h, ITY)), dim3(256), 0, ctx->stream, w, h, 1.0f / sigma,
                      T, mpb, M, (size_t)pitch);
   DMSC_HIP(hipGetLastError());

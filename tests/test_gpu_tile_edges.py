@@ -223,3 +223,24 @@ def test_resident_block_filter(ctx, w, h):
         assert got[2] == out[0][2]
         np.testing.assert_array_equal(got[0], out[0][0])
         np.testing.assert_array_equal(got[1], out[0][1])
+
+
+# a context's first affinities inside a captured graph, replayed on new inputs
+@pytest.mark.parametrize("w,h", [(9, 12), (70, 45)])
+def test_affinities_in_a_graph(w, h):
+    print(f"case: captured affinities {w}x{h}", flush=True)
+    s = torch.cuda.Stream()
+    c = dm.Context(stream=s)
+    pb = torch.zeros(h, w, device="cuda")
+    g = torch.cuda.CUDAGraph()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(g, stream=s):
+        m = c.intervene(pb)
+    for seed in range(3):
+        pb.copy_(torch.from_numpy(np.random.RandomState(seed).rand(h, w).astype(np.float32)))
+        torch.cuda.synchronize()
+        g.replay()
+        eager = c.intervene(pb)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(bits(host(m)), bits(host(eager)))
+    c.close()
