@@ -321,7 +321,7 @@ __global__ void k_lz_slots(unsigned long long* slots, int count, unsigned* z, in
 // for every vector and wait for two launches: 16.8 us a step.  Here every
 // block stays resident, so each lane keeps its row's 81 matrix entries, its z
 // and its last q in registers and a step moves the stencil halo of z, the
-// basis row and two partial sums per block: 6.3 us, bound by the two
+// basis row and two partial sums per block: 5.9 us, bound by the two
 // exchanges (about 3,800 cycles each of 15,000) and the 81 LDS reads per row
 // (3,500).
 //  * Rows are consecutive, so halo and sums keep the linear indexing and the

@@ -401,12 +401,7 @@ __device__ __forceinline__ void corner_sum(const uint32_t (&pk)[8][16], int i0, 
                         : 0u;
 }
 
-// chi^2 of one split of the half-disc pair from the packed corner counts:
-// a = c[i0] - c[i1] + c[i2] - c[i3], b = c[j0] - c[j1] + c[j2] - c[j3] per
-// bin (uint16 modulo arithmetic recovers the exact counts), optional bin
-// blur, normalisation to sum 8 and 0.5 * sum (a-b)^2/(a+b) with the
-// reference's 32-slot tree sums (rotate.cu:352-472).
-// Divisions: n / s for the values that occur here (0 or n in [2^-80, 2^7], s
+// n / s for the values that occur in chi^2 (0 or n in [2^-80, 2^7], s
 // in [2^-17, 2^10]), where no scaling is needed: Newton steps with fused
 // multiply-adds from the hardware reciprocal, whose last correction rounds
 // correctly (Markstein, IBM J. Res. Dev. 34, 1990), so the quotient is the
@@ -420,6 +415,11 @@ __device__ __forceinline__ float div_exact(float n, float s) {
   return fmaf(fmaf(-s, q, n), r, q);
 }
 
+// chi^2 of one split of the half-disc pair from the packed corner counts:
+// a = c[i0] - c[i1] + c[i2] - c[i3], b = c[j0] - c[j1] + c[j2] - c[j3] per
+// bin (uint16 modulo arithmetic recovers the exact counts), optional bin
+// blur, normalisation to sum 8 and 0.5 * sum (a-b)^2/(a+b) with the
+// reference's 32-slot tree sums (rotate.cu:352-472).
 // PAIR: the pixel's 64 bins are split over this lane (32 bins in pk) and
 // its neighbour lane (lane ^ 1); each 32-slot tree sum is completed with the
 // partner's as lo + hi (rotate.cu:384-389 adds slot 32 to slot 0), and IEEE
