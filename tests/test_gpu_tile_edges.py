@@ -244,3 +244,18 @@ def test_affinities_in_a_graph(w, h):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(bits(host(m)), bits(host(eager)))
     c.close()
+
+
+# thinning: windows of 64 x 64 pixels for 32 x 32, two iterations per launch
+@pytest.mark.parametrize("w,h,fill", [(6, 6, 1.0), (32, 33, 1.0), (65, 40, 0.6), (130, 97, 0.85), (96, 128, 1.0)])
+def test_thinning_windows(ctx, w, h, fill):
+    print(f"case: thinning {w}x{h}, {fill}", flush=True)
+    r = np.random.RandomState(w)
+    nm = (r.rand(h, w) < fill).astype(np.float32)  # up to a solid block: many iterations
+    g = (0.1 + 0.9 * r.rand(h, w)).astype(np.float32)
+    got, thin, it = ctx.postprocess(ctx.upload(g), ctx.upload(nm))
+    rg, rthin, rit = O.postprocess(g, nm)
+    assert it == rit
+    assert np.array_equal(host(thin) == host(thin).min(), rthin == rthin.min())
+    np.testing.assert_allclose(host(thin), rthin, rtol=0, atol=1e-6)
+    np.testing.assert_allclose(host(got), rg, rtol=0, atol=1e-6)
