@@ -105,9 +105,9 @@ extern int lanczos_trace;
 // Rows per block of the Lanczos SpMV step kernel: 0 = automatic (256 for the
 // two-kernel steps, 512 for the fused mixed step), or 64, 256, 512.
 extern int lanczos_k1_threads;
-// Plain steps in one resident launch per check: most rounds of reads of an
-// awaited value before the launch is given up for two kernels per step (0 =
-// always two kernels).
+// Resident launches (plain steps of a check period, block filter of an outer
+// iteration): most rounds of reads of an awaited value before the launch is
+// given up for launches per step (0 = always those).
 extern int resident_polls;
 // Mixed eigensolver step: 2 = one fused kernel per step over pixel tiles
 // (default), 1 = one fused kernel over runs of consecutive rows (when

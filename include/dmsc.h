@@ -237,11 +237,13 @@ int dmsc_write_pgm(const char* path, int w, int h, const float* h_data);
  *                         kernel: 0 = automatic (default: 256 for two-kernel
  *                         steps, 512 for the fused mixed step), 64, 256 or
  *                         512 (512 applies to the fused step only).
- *   "resident_polls":  plain eigensolver: how often a block of the launch
- *                         that runs a whole check period looks for another
- *                         block's value before the solve starts over with
- *                         two kernels per step (0-2^20, 16384; 0 = always
- *                         two kernels; results are identical).
+ *   "resident_polls":     the launches whose blocks wait for each other (a
+ *                         check period of the plain eigensolver, an outer
+ *                         iteration's filter of the block eigensolver): how
+ *                         often a block looks for another's value before the
+ *                         work is done again with launches per step (0-2^20,
+ *                         16384; 0 = always launches per step, for a GPU that
+ *                         several processes share; results are identical).
  *   "lanczos_mixed_fused": mixed eigensolver step as one kernel staging the
  *                         basis vector in LDS, over pixel tiles (2, default)
  *                         or runs of consecutive rows (1, when the stencil
