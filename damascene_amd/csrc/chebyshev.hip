@@ -649,8 +649,14 @@ __global__ __launch_bounds__(256) void k_cheb_resid_sum(int nblk, const double* 
 // threads each; thread j sums the partials of blocks j, j + 16, ... in
 // order, then the 16 sums are added in a fixed tree (deterministic).
 constexpr int kGramSumSplit = 16;
+// The sums go straight to pinned host memory (24 KB), as do the residuals of
+// k_cheb_resid_sum and the stall flag of the filter's launch: each copy back
+// costs an outer iteration a launch and the gap before it (solve and spectral Pb
+// at 160x120: 3.17 ms against 3.36 with two copies back and two up).
 __global__ __launch_bounds__(1024) void k_cheb_gram_sum(int nblk, const double* __restrict__ part,
-                                                        double* __restrict__ gram) {
+                                                        double* __restrict__ gram, const int* __restrict__ stalled,
+                                                        int* __restrict__ host_stalled) {
+  if (blockIdx.x == 0 && threadIdx.x == 0 && stalled) *host_stalled = *stalled;
   __shared__ double red[kGramSumSplit][64];
   const int el = threadIdx.x & 63, j = threadIdx.x >> 6;
   const int e = blockIdx.x * 64 + el;
@@ -1182,11 +1188,10 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
   const int nblk = div_up(n, chunk);
   const size_t blk = (size_t)kPlanes * vs * sizeof(float4);
   const int nrb = div_up(n, 256);  // k_cheb_resid_rotate blocks
-  const size_t o_part = 4 * blk, o_gram = o_part + (size_t)kGrams * nblk * kB * kB * sizeof(double),
-               o_rot = o_gram + ((size_t)kGrams * kB * kB + 2) * sizeof(double),  // with the launch's stall flag
+  const size_t o_part = 4 * blk, o_stall = o_part + (size_t)kGrams * nblk * kB * kB * sizeof(double),
+               o_rot = o_stall + 2 * sizeof(double),
                o_theta = o_rot + (size_t)kB * kB * sizeof(double),
-               o_res = o_theta + (size_t)kResidMax * sizeof(double),
-               o_rpart = o_res + (size_t)kResidMax * sizeof(double),
+               o_rpart = o_theta + (size_t)kResidMax * sizeof(double),
                bytes = o_rpart + (size_t)nrb * kResidMax * sizeof(double);
   void* base;
   DMSC_TRY(ctx->scratch(3, bytes, &base));
@@ -1194,13 +1199,12 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
   float4* X0 = (float4*)Bp;
   float4* ring[3] = {(float4*)(Bp + blk), (float4*)(Bp + 2 * blk), (float4*)(Bp + 3 * blk)};
   double* part = (double*)(Bp + o_part);
-  double* gram = (double*)(Bp + o_gram);
   double* rot = (double*)(Bp + o_rot);
   double* d_theta = (double*)(Bp + o_theta);
-  double* d_res = (double*)(Bp + o_res);
   double* rpart = (double*)(Bp + o_rpart);
   int* pin;
   DMSC_TRY(ctx->pinned(&pin));
+  // written by the device and read by the host after it has synchronised
   double* h_gram = (double*)((char*)pin + kPinGram);
   double* h_rot = (double*)((char*)pin + kPinRot);
   double* h_theta = (double*)((char*)pin + kPinTheta);
@@ -1230,8 +1234,8 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
   std::unique_ptr<ResidentGrid> gate;
   if (rs.units) gate = std::make_unique<ResidentGrid>(ctx->device);
   bool whole = gate && gate->held();
-  int* stalled = (int*)(gram + (size_t)kGrams * kB * kB);
-  const int* h_stalled = (const int*)(h_gram + (size_t)kGrams * kB * kB);
+  int* stalled = (int*)(Bp + o_stall);
+  int* h_stalled = (int*)(h_gram + (size_t)kGrams * kB * kB);
   RunCoefs co;
   for (int outer = 0; outer < kMaxOuter; outer++) {
     // scaled Chebyshev filter of degree deg damping [cut, kUpper], normalised at 0
@@ -1265,8 +1269,9 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
     float4* Wb = ring[(cur + 1) % 3];
     DMSC_TRY(product_f64(shape, s, w, h, A, pitchz, Y, Wb, vs));
     hipLaunchKernelGGL(k_cheb_gram, dim3(nblk), dim3(256), 0, s, n, vs, chunk, Y, Wb, X0, part);
-    hipLaunchKernelGGL(k_cheb_gram_sum, dim3(div_up(kGrams * kB * kB, 64)), dim3(1024), 0, s, nblk, part, gram);
-    DMSC_HIP(hipMemcpyAsync(h_gram, gram, kGrams * kB * kB * sizeof(double) + sizeof(int), hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(k_cheb_gram_sum, dim3(div_up(kGrams * kB * kB, 64)), dim3(1024), 0, s, nblk, part, h_gram,
+                       whole ? stalled : nullptr, h_stalled);
+    DMSC_HIP(hipGetLastError());
     // one host round trip per outer iteration: the Gram matrices of this
     // block and the residuals of the previous Ritz pairs (enqueued last
     // iteration, read here)
@@ -1327,16 +1332,16 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
     // the rotation S and the wanted Ritz values go to the device either way
     std::memcpy(h_rot, S.data(), sizeof(double) * kB * kB);
     for (int j = 0; j < nvec; j++) h_theta[j] = theta[j];
-    DMSC_HIP(hipMemcpyAsync(rot, h_rot, sizeof(double) * kB * kB, hipMemcpyHostToDevice, s));
-    DMSC_HIP(hipMemcpyAsync(d_theta, h_theta, sizeof(double) * nvec, hipMemcpyHostToDevice, s));
+    // (one copy: theta follows the rotation on both sides)
+    static_assert(kPinTheta == kPinRot + sizeof(double) * kB * kB, "the Ritz values follow the rotation");
+    DMSC_HIP(hipMemcpyAsync(rot, h_rot, sizeof(double) * (kB * kB + nvec), hipMemcpyHostToDevice, s));
     // residual |A y_j - theta_j y_j| of each wanted Ritz vector y_j = Y s_j,
     // formed per pixel on the device by the pass that writes the rotated
     // block (the next filter input, or the output when the solve stops
-    // here); read back at the next round trip (or below, at a stop)
+    // here); read by the host at the next round trip (or below, at a stop)
     hipLaunchKernelGGL(k_cheb_resid_rotate, dim3(nrb), dim3(256), 0, s, n, vs, Y, Wb, rot, d_theta, nvec, rpart,
                        rule ? nvec : -1, rule ? nullptr : X0, rule ? d_out : nullptr);
-    hipLaunchKernelGGL(k_cheb_resid_sum, dim3(nvec), dim3(256), 0, s, nrb, rpart, d_res);
-    DMSC_HIP(hipMemcpyAsync(h_res, d_res, sizeof(double) * nvec, hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(k_cheb_resid_sum, dim3(nvec), dim3(256), 0, s, nrb, rpart, h_res);
     if (rule) {
       DMSC_HIP(hipGetLastError());
       DMSC_HIP(hipStreamSynchronize(s));
