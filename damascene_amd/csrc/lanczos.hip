@@ -335,7 +335,9 @@ __global__ void k_lz_slots(unsigned long long* slots, int count, unsigned* z, in
 //    publishes exchange e + 1 only after it has seen all of e, so whoever has
 //    all of e + 1 knows that e is read everywhere.  Slots alternate between
 //    two sets per sum, z between z0 and z1.  Emptied values have arrived
-//    (drain_memory) before the partial that lets others look at them.
+//    (drain_memory) before the partial that lets others look at them: an
+//    alpha slot before the same step's beta partial, a beta slot and z before
+//    the next step's alpha partial.
 //  * Reads that come too early delay the stores they wait for: a first look
 //    1,024 cycles after the store takes 3,700 cycles for the sum against
 //    6,500 at once.
@@ -474,6 +476,7 @@ __global__ __launch_bounds__(kRunRows) void k_lz_run(LzBufs b, int w, int halo, 
       }
       __builtin_amdgcn_s_sleep(16);  // in units of 64 cycles
       const float alpha = (float)sum_slots(sla);
+      drain_memory();  // the emptied alpha slot, before this step's beta partial (both long since arrived)
       if (lane == 0) coef[0] = alpha;
     }
     __syncthreads();
