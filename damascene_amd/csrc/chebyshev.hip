@@ -901,16 +901,18 @@ __global__ __launch_bounds__(64 * U, U > 8 ? 3 : 2) void k_cheb_run(int w, int h
       v[u] = __builtin_amdgcn_raw_buffer_load_b128(src, list[frame_entry(u)][1] + (unsigned)j * plane, hf * 4 * plane,
                                                    kDeviceScope | kVolatile);
   };
+  // false: given up.  The caller sets quit, and only between the two barriers
+  // of a half: before the first a slow wave may still stand at the test of
+  // quit that ends the half before.
   const auto await_frame = [&](u32x4 (&v)[kItems], int hf, int k) {
     for (int i = 0;; i++) {
       bool all = true;
 #pragma unroll
       for (int u = 0; u < kItems; u++) all = all && max(max(v[u].x, v[u].y), max(v[u].z, v[u].w)) != kRunNone;
-      if (all) break;
+      if (all) return true;
       if (i >= polls || ((i & 63) == 63 && resident::shared_load(stalled))) {
         resident::shared_store(stalled, 1);
-        quit = 1;
-        break;
+        return false;
       }
       __builtin_amdgcn_s_sleep(1);
       load_frame(v, hf, k);
@@ -925,17 +927,19 @@ __global__ __launch_bounds__(64 * U, U > 8 ? 3 : 2) void k_cheb_run(int w, int h
     const unsigned soff = hf * 4 * plane;
     Frame late;
     u32x4(&v)[kItems] = kEarly ? early.v : late.v;
-    if (kEarly) await_frame(v, hf, k);
+    bool complete = true;
+    if (kEarly) complete = await_frame(v, hf, k);
     __syncthreads();  // the last half's reads are over
 #pragma unroll
     for (int r = 0; r < 4; r++)
       if (mine >> r & 1) s0[(r + 5) * kRunSW * 4] = held[hf][r];
     if (!kEarly) {
       load_frame(v, hf, k);
-      await_frame(v, hf, k);
+      complete = await_frame(v, hf, k);
     }
+    if (!complete) quit = 1;
 #pragma unroll
-      for (int u = 0; u < kItems; u++) ((u32x4*)sx)[list[frame_entry(u)][0] * 4 + j] = v[u];
+    for (int u = 0; u < kItems; u++) ((u32x4*)sx)[list[frame_entry(u)][0] * 4 + j] = v[u];
     __syncthreads();
     if (quit) return false;
     // the next step's entries still hold those of three steps before; all have

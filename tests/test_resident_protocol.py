@@ -1,5 +1,6 @@
-"""The order of waits, barriers and stores in the kernel whose blocks hand
-each other values while they run (k_lz_run), read from its source.
+"""The order of waits, barriers and stores in the kernels whose blocks hand
+each other values while they run (k_lz_run, k_cheb_run), read from their
+source.
 
 A place that others wait on is emptied before it is used again.  Another block
 may look at it once that block has awaited a value published later in the
@@ -96,3 +97,15 @@ def test_lanczos_emptied_after_all_have_read():
     assert step.index("empty_b") > step.index("wait_a")
     assert step.index("empty_z") > step.index("wait_a")
     assert step.index("wait_b") > step.index("put_b") and step.index("wait_z") > step.index("put_z")
+
+
+def test_filter_gives_up_between_barriers():
+    """A wave leaves at `if (quit)` behind a barrier; nothing may set quit
+    before every wave has passed that test, which the next barrier shows."""
+    half = kernel_body("chebyshev.hip", "k_cheb_run", "const auto half =")
+    await_frame = kernel_body("chebyshev.hip", "k_cheb_run", "const auto await_frame =")
+    sets = r"\bquit = 1" + (r"|await_frame\(" if "quit" in await_frame else "")
+    where = [m.start() for m in re.finditer(sets, half)]
+    first_barrier, last_barrier = half.index("__syncthreads()"), half.rindex("__syncthreads()")
+    assert where and all(first_barrier < i < last_barrier for i in where)
+    assert half.index("if (quit) return") > last_barrier
