@@ -28,7 +28,7 @@ HIP_FLAGS = COMMON + [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-builtin", "-I", CSRC,
               "-I", os.path.join(ROOT, "include"), "-Wall"]
 
-HOST_ONLY = ["tables.cpp", "generator.cpp", "symeig.cpp", "walks.cpp"]
+HOST_ONLY = ["tables.cpp", "generator.cpp", "symeig.cpp"]
 # host files with no oracle parity to keep: optimised harder (the block
 # solver's Rayleigh-Ritz step sits between GPU launches)
 HOST_FAST = {"symeig.cpp": ["-O3", "-ffp-contract=fast", "-fno-math-errno", "-fbuiltin"]}

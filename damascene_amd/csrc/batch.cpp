@@ -39,10 +39,6 @@ int make_lanes(Ctx* ctx, int lanes) {
     c->stream = s;
     c->own_stream = true;
     c->overlap_stages = false;
-    if (const int rc = init_walks(c); rc != DMSC_OK) {
-      delete c;
-      return rc;
-    }
     ctx->lanes.push_back(c);
   }
   return DMSC_OK;

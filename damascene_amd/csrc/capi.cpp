@@ -41,8 +41,6 @@ Ctx::~Ctx() {
   for (int i = 0; i < kArenas; i++)
     if (arena[i]) (void)hipFree(arena[i]);
   if (d_texton_coeffs) (void)hipFree(d_texton_coeffs);
-  for (uint8_t* t : d_walks)
-    if (t) (void)hipFree(t);
   if (h_pinned) (void)hipHostFree(h_pinned);
   for (hipEvent_t e : aux_ev)
     if (e) (void)hipEventDestroy(e);
@@ -138,10 +136,6 @@ int dmsc_ctx_create(dmsc_ctx** out, int device, void* stream) {
   // want a private stream create one and pass it in
   c->stream = (hipStream_t)stream;
   c->own_stream = false;
-  if (const int rc = init_walks(c); rc != DMSC_OK) {
-    delete c;
-    return rc;
-  }
   *out = c;
   return DMSC_OK;
 }
@@ -592,7 +586,7 @@ int dmsc_calc_gpb(dmsc_ctx* ctx, int npix, int pitch, int norient, const float* 
 int dmsc_intervene(dmsc_ctx* ctx, int w, int h, const float* mpb, float* M, int pitch, float sigma) {
   CHECK_CTX(ctx);
   DMSC_ARG(w > 5 && h > 5 && pitch >= w * h && mpb && M && sigma > 0, "bad arguments");
-  return launch_intervene(ctx, w, h, mpb, M, pitch, sigma);
+  return launch_intervene(ctx->stream, w, h, mpb, M, pitch, sigma);
 }
 
 int dmsc_convert_matrix(dmsc_ctx* ctx, int w, int h, float* M, int pitch, float* dsum, float* rs) {
@@ -859,7 +853,7 @@ int dmsc_gpb(dmsc_ctx* ctx, int w, int h, const uint32_t* rgb, const dmsc_gpb_pa
   DMSC_TRY(launch_nonmax(s, w, h, mpb, pitch, spb, (int*)all, nmax));  // spb/all as scratch here
   if (timing) DMSC_HIP(hipEventRecord(ev[3], s));
   // damascene.cu:417-420 intervene
-  DMSC_TRY(launch_intervene(ctx, w, h, nmax, mat, pitch, 0.1f));
+  DMSC_TRY(launch_intervene(s, w, h, nmax, mat, pitch, 0.1f));
   if (timing) DMSC_HIP(hipEventRecord(ev[4], s));
   // damascene.cu:433 generalizedEigensolve
   DMSC_TRY(run_eigensolve(ctx, w, h, mat, pitch, p.n_eig, p.tol, p.precision, out->h_eigvals, vec,

@@ -32,7 +32,6 @@ struct Ctx {
   void* arena[kArenas] = {};
   size_t arena_bytes[kArenas] = {};
   float* d_texton_coeffs = nullptr;
-  uint8_t* d_walks[2] = {nullptr, nullptr};  // intervening-contour tables (intervening.hip), by `narrow`
   int* h_pinned = nullptr;  // pinned host block (64 KiB) for asynchronous read-backs
   hipStream_t aux = nullptr;  // second stream (default priority) for work overlapped with `stream`
   hipEvent_t aux_ev[2] = {};

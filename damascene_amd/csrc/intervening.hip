@@ -14,12 +14,15 @@
 //    values.
 //  * The pixels crossed are the same for every pixel whose window is not
 //    clipped: their offsets are compiled into the kernel (418 reads for the 80
-//    points).  Near the image's edges 36 points have a second set, and
-//    some none: a table by the window's reaches tells which.
+//    points).  Near the image's edges 36 points have a second set: a constant
+//    per point, with a bit for each pair of the window's reaches, tells when.
+//    The launch needs no table in memory, so nothing is allocated or copied
+//    for it and a caller may capture it.
 //  * A thread takes both walks of each of its entries and writes the
 //    symmetrised value once: no clearing, no second kernel.
-// It takes 31 us at 640x480 (100 MB written) and 22 us at 160x120 (140 us
-// before), where most waves touch an edge and wait on the table.
+// It takes 27 us at 640x480 (100 MB written) and 15 us at 160x120 (140 us
+// before), where most waves touch an edge; with a table in memory of the set
+// each clipped window takes, waves waited on it: 30 and 18 us.
 #include <utility>
 
 #include "dmsc_device.hpp"
@@ -65,21 +68,21 @@ struct Pixel {
   uint32_t g0;  // g(0): nothing crossed
 };
 
-__device__ __forceinline__ int reach(int i, int n) { return min(i, 5) * 6 + min(n - 1 - i, 5); }
-
-// Affinity of the walk from the pixel (x, y), at b, to point D, any window.
+// Affinity (its bits) of the walk from the pixel (x, y), at b, to point D
+// inside its window, which may be clipped.
 template <int D>
-__device__ __forceinline__ float any_walk(const uint32_t* b, int x, int y, const Pixel& P,
-                                          const uint8_t* __restrict__ codes) {
-  const int code = codes[(reach(y, P.h) * kReaches + reach(x, P.w)) * kWalkArea + D];
+__device__ __forceinline__ uint32_t any_walk(const uint32_t* b, int x, int y, const Pixel& P) {
   uint32_t g = walk_min<false, D>(b, P.g0);
-  if constexpr (kSecondWalks.n[D] >= 0) g = code == 2 ? walk_min<true, D>(b, P.g0) : g;
-  return code ? __uint_as_float(g) : 0.0f;
+  if constexpr (constexpr uint32_t kSecond = kWalkRules.second[D]; kSecond != 0) {
+    const int at = walk_bit(D, walk_reach(walk_dy(D), y, P.h), walk_reach(walk_dx(D), x, P.w));
+    if (__builtin_amdgcn_ubfe(kSecond, at, 1)) g = walk_min<true, D>(b, P.g0);
+  }
+  return g;
 }
 
 // M(p, p + D): the mean of the two walks, 0 past the image.
 template <int D, bool FULL>
-__device__ __forceinline__ float entry(const Pixel& P, const uint8_t* __restrict__ T) {
+__device__ __forceinline__ float entry(const Pixel& P) {
   constexpr int dy = walk_dy(D), dx = walk_dx(D), R = kWalkArea - 1 - D;  // R: the way back
   if constexpr (dy == 0 && dx == 0) {
     return 1.0f;
@@ -91,29 +94,27 @@ __device__ __forceinline__ float entry(const Pixel& P, const uint8_t* __restrict
     } else {
       const int x = P.x + dx, y = P.y + dy;
       const bool in = x >= 0 && y >= 0 && x < P.w && y < P.h;
-      // past the image the way back starts nowhere: read from the pixel itself
-      const float there = any_walk<D>(P.b, P.x, P.y, P, T);
-      const float back = any_walk<R>(q, in ? x : P.x, in ? y : P.y, P, T);
+      const float there = __uint_as_float(any_walk<D>(P.b, P.x, P.y, P));
+      const float back = __uint_as_float(any_walk<R>(q, x, y, P));
       return in ? 0.5f * (there + back) : 0.0f;
     }
   }
 }
 
 template <bool FULL, int... D>
-__device__ __forceinline__ void entries(const Pixel& P, const uint8_t* __restrict__ T, float* __restrict__ M, size_t pitch, bool live,
+__device__ __forceinline__ void entries(const Pixel& P, float* __restrict__ M, size_t pitch, bool live,
                                         std::integer_sequence<int, D...>) {
   if constexpr (FULL) {
-    ((M[(size_t)D * pitch] = entry<D, true>(P, T)), ...);
+    ((M[(size_t)D * pitch] = entry<D, true>(P)), ...);
   } else {
     auto put = [&](int d, float v) {
       if (live) M[(size_t)d * pitch] = v;
     };
-    (put(D, entry<D, false>(P, T)), ...);
+    (put(D, entry<D, false>(P)), ...);
   }
 }
 
-__global__ __launch_bounds__(256) void k_affinities(int w, int h, float rs, const uint8_t* __restrict__ T,
-                                                    const float* __restrict__ mpb,
+__global__ __launch_bounds__(256) void k_affinities(int w, int h, float rs, const float* __restrict__ mpb,
                                                     float* __restrict__ M, size_t pitch) {
   // the way back from a point past the tile's frame is formed and dropped:
   // five rows and columns of slack on each side
@@ -139,8 +140,8 @@ __global__ __launch_bounds__(256) void k_affinities(int w, int h, float rs, cons
   // no window of the pixel's or its disc points' is clipped
   const bool full = x >= 10 && y >= 10 && x < w - 10 && y < h - 10;
   constexpr std::make_integer_sequence<int, kWalkArea> all;
-  if (__all(full)) entries<true>(P, T, row, pitch, live, all);
-  else entries<false>(P, T, row, pitch, live, all);
+  if (__all(full)) entries<true>(P, row, pitch, live, all);
+  else entries<false>(P, row, pitch, live, all);
   if (blockIdx.x == 0 && blockIdx.y == 0) {  // the columns past the image
     const size_t n = (size_t)w * h, pad = pitch - n;
     for (size_t i = threadIdx.x; i < kWalkArea * pad; i += 256) M[i / pad * pitch + n + i % pad] = 0.0f;
@@ -149,22 +150,9 @@ __global__ __launch_bounds__(256) void k_affinities(int w, int h, float rs, cons
 
 }  // namespace
 
-// A context's device copies of the walk codes, uploaded when it is made: the
-// launch itself allocates and copies nothing, so a caller may capture it.
-int init_walks(Ctx* ctx) {
-  for (int narrow = 0; narrow < 2; narrow++) {
-    const std::vector<uint8_t>& c = walk_codes(narrow != 0);
-    if (c.empty()) return fail(DMSC_ERR_INTERNAL, "a clipped window crosses an unexpected set of pixels");
-    DMSC_HIP(hipMalloc(&ctx->d_walks[narrow], c.size()));
-    DMSC_HIP(hipMemcpy(ctx->d_walks[narrow], c.data(), c.size(), hipMemcpyHostToDevice));
-  }
-  return DMSC_OK;
-}
-
-int launch_intervene(Ctx* ctx, int w, int h, const float* mpb, float* M, int pitch, float sigma) {
-  const uint8_t* T = ctx->d_walks[w < 11 || h < 11];
-  hipLaunchKernelGGL(k_affinities, dim3(div_up(w, ITX), div_up(h, ITY)), dim3(256), 0, ctx->stream, w, h, 1.0f / sigma,
-                     T, mpb, M, (size_t)pitch);
+int launch_intervene(hipStream_t s, int w, int h, const float* mpb, float* M, int pitch, float sigma) {
+  hipLaunchKernelGGL(k_affinities, dim3(div_up(w, ITX), div_up(h, ITY)), dim3(256), 0, s, w, h, 1.0f / sigma, mpb, M,
+                     (size_t)pitch);
   DMSC_HIP(hipGetLastError());
   return DMSC_OK;
 }

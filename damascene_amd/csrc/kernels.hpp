@@ -51,8 +51,7 @@ int launch_calc_gpb(hipStream_t s, int n, int pitch, int norient, const float* c
                     const float* mpb, float* all, float* gpb);
 
 // ------------------------------------------------------------- affinity / stencil
-int init_walks(Ctx* ctx);  // its tables, when the context is made
-int launch_intervene(Ctx* ctx, int w, int h, const float* mpb, float* M, int pitch, float sigma);
+int launch_intervene(hipStream_t s, int w, int h, const float* mpb, float* M, int pitch, float sigma);
 
 struct StencilOffsets {
   int off[kStencilArea];          // cumulative linear offset of each diagonal

@@ -1,23 +1,21 @@
 // walks.hpp -- which pixels the intervening-contour walks cross
-// (intervening.cu:44-475), as tables built once.
+// (intervening.cu:44-475), as constants.
 //
 // The reference walks Bresenham lines from a pixel to every point of the
 // boundary of its 11 x 11 window (clipped to the image) and records, for the
 // disc points a walk is the best integer approximant of, the affinity of the
 // strongest boundary crossed so far; later walks replace earlier ones.
 // Which pixels are crossed on the way to a disc point depends only on how
-// far the window reaches to the four sides, so the walks are followed here
-// once per reach, by the compiler for the full window and on the host for
-// the clipped ones.
+// far the window reaches to the four sides, so the compiler follows the walks
+// once per reach.
 #pragma once
 #include <cstdint>
-#include <vector>
+#include <utility>
 
 namespace dmsc {
 
 constexpr int kWalkArea = 81;   // points of the radius-5 disc, raster order
 constexpr int kMaxCross = 13;   // distinct pixels crossed on the way to one
-constexpr int kReaches = 36;    // (reach to one side, to the other), each 0..5
 
 constexpr int walk_half_width(int dy) {
   return dy == 0 ? 5 : (dy >= -3 && dy <= 3) ? 4 : (dy == 4 || dy == -4) ? 3 : 0;
@@ -165,12 +163,63 @@ constexpr Walks second_walks() {
 }
 constexpr Walks kSecondWalks = second_walks();
 
-// Which set point d takes for a window, at [(row reach * 36 + column reach) *
-// 81 + d] (a reach is 6 * to the lower side + to the upper): 0 no affinity, 1
-// the full window's, 2 the second.  Images of at least 11 pixels a side have
-// windows that are full to one side of each axis, and the table holds those
-// 121; a `narrow` image's holds all 1,296.  Empty if some window had a third
-// set.
-const std::vector<uint8_t>& walk_codes(bool narrow);
+// A walk speaks for exactly the points inside the window, and which set a point
+// d takes depends only on how far the window reaches towards it: in x and y
+// each the reach to the point's side, or where that component is 0 the smaller
+// of both reaches.  Bit walk_bit(d, reach in y, reach in x) of second[d] is set
+// where d takes the second set.
+struct WalkRules {
+  uint32_t second[kWalkArea] = {};
+  bool as_described = true;  // of every window, and no window had a third set
+};
+// In 0..29 where the point is inside the window.
+constexpr int walk_bit(int d, int ry, int rx) { return walk_dy(d) ? 6 * (ry - 1) + rx : 6 * (rx - 1) + ry; }
+
+// The rules of the points on one side in x and y (a component of 0 counts as
+// negative), for windows that reach ry towards it in y.
+template <int SX, int SY, int RY>
+constexpr WalkRules quarter_rules() {
+  WalkRules R;
+  for (int rx = 0; rx < 6; rx++) {
+    const Walks W = window_walks(SX < 0 ? rx : 5, SX < 0 ? 5 : rx, SY < 0 ? RY : 5, SY < 0 ? 5 : RY);
+    for (int d = 0; d < kWalkArea; d++) {
+      const int dx = walk_dx(d), dy = walk_dy(d);
+      if ((dx > 0) != (SX > 0) || (dy > 0) != (SY > 0) || d == kWalkArea / 2) continue;
+      const bool inside = rx >= (dx < 0 ? -dx : dx) && RY >= (dy < 0 ? -dy : dy);
+      R.as_described = R.as_described && (W.n[d] >= 0) == inside;
+      if (!inside || same_walk(W, kFullWalks, d)) continue;
+      R.as_described = R.as_described && same_walk(W, kSecondWalks, d);
+      R.second[d] |= 1u << walk_bit(d, RY, rx);
+    }
+  }
+  return R;
+}
+template <int SX, int SY, int RY>
+constexpr WalkRules kQuarterRules = quarter_rules<SX, SY, RY>();  // each within a compiler's step limit
+
+constexpr void add_rules(WalkRules& R, const WalkRules& Q) {
+  for (int d = 0; d < kWalkArea; d++) R.second[d] |= Q.second[d];
+  R.as_described = R.as_described && Q.as_described;
+}
+template <int SX, int SY, int... RY>
+constexpr void add_quarter(WalkRules& R, std::integer_sequence<int, RY...>) {
+  (add_rules(R, kQuarterRules<SX, SY, RY>), ...);
+}
+constexpr WalkRules walk_rules() {
+  WalkRules R;
+  add_quarter<-1, -1>(R, std::make_integer_sequence<int, 6>());
+  add_quarter<1, -1>(R, std::make_integer_sequence<int, 6>());
+  add_quarter<-1, 1>(R, std::make_integer_sequence<int, 6>());
+  add_quarter<1, 1>(R, std::make_integer_sequence<int, 6>());
+  return R;
+}
+constexpr WalkRules kWalkRules = walk_rules();
+static_assert(kWalkRules.as_described, "a clipped window's walks");
+
+// The window's reach towards side `d` (a point's component) of position i of n.
+constexpr int walk_reach(int d, int i, int n) {
+  const int lo = i < 5 ? i : 5, hi = n - 1 - i < 5 ? n - 1 - i : 5;
+  return d < 0 ? lo : d > 0 ? hi : lo < hi ? lo : hi;
+}
 
 }  // namespace dmsc

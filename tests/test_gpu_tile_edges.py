@@ -259,3 +259,27 @@ def test_thinning_windows(ctx, w, h, fill):
     assert np.array_equal(host(thin) == host(thin).min(), rthin == rthin.min())
     np.testing.assert_allclose(host(thin), rthin, rtol=0, atol=1e-6)
     np.testing.assert_allclose(host(got), rg, rtol=0, atol=1e-6)
+
+
+# a context made while another stream is captured in the global mode (as
+# torch captures), and used once the capture has ended
+def test_context_made_during_a_capture(ctx):
+    print("case: context made during a capture", flush=True)
+    other = torch.cuda.Stream()
+    s = torch.cuda.Stream()
+    x = torch.zeros(1000, device="cuda")
+    pb = torch.from_numpy(np.random.RandomState(5).rand(40, 33).astype(np.float32)).cuda()
+    g = torch.cuda.CUDAGraph()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(g, stream=s):
+        x.add_(1.0)
+        c = dm.Context(stream=other)
+        x.add_(1.0)
+    for turn in range(1, 4):
+        g.replay()
+        torch.cuda.synchronize()
+        assert float(x.sum()) == 2000.0 * turn
+        m = c.intervene(pb)
+        c.synchronize()
+        np.testing.assert_array_equal(bits(host(m)), bits(host(ctx.intervene(pb))))
+    c.close()
