@@ -6,6 +6,7 @@ import torch
 
 import damascene_amd as dm
 from damascene_amd import autograd as AG
+from damascene_amd._lib import check, lib
 from oracle import grad_ref as G
 from oracle import pyoracle as O
 
@@ -283,3 +284,37 @@ def test_context_made_during_a_capture(ctx):
         c.synchronize()
         np.testing.assert_array_equal(bits(host(m)), bits(host(ctx.intervene(pb))))
     c.close()
+
+
+# matrices whose rows are padded: up to 4,096 columns past the image cleared by
+# its own blocks, more by a launch of their own
+@pytest.mark.parametrize("w,h,pad", [(6, 6, 4), (33, 21, 4096), (33, 21, 4100), (640, 480, 307200)])
+def test_affinity_padding(ctx, w, h, pad):
+    n = w * h
+    pitch = n + pad
+    print(f"case: affinity {w}x{h}, pitch {pitch}", flush=True)
+    pb = ctx.upload(np.random.RandomState(w).rand(h, w).astype(np.float32))
+    ref = ctx.intervene(pb)
+
+    def call(m):
+        check(lib().dmsc_intervene(ctx.handle, w, h, pb.data_ptr(), m.data_ptr(), m.shape[1], 0.1))
+
+    m = torch.full((81, pitch), 7.0, device="cuda")
+    call(m)
+    assert torch.equal(m[:, :n], ref[:, :n]) and not bool(m[:, n:].any())
+
+    def us(m, reps=10):
+        call(m)
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        for _ in range(reps):
+            call(m)
+        e[1].record()
+        torch.cuda.synchronize()
+        return e[0].elapsed_time(e[1]) / reps * 1e3
+
+    if n > 100000:
+        tight, wide = us(torch.empty_like(ref)), us(m)
+        print(f"{tight:.0f} us at pitch {ref.shape[1]}, {wide:.0f} us at {pitch}", flush=True)
+        # twice the bytes written; ten times leaves room for any launch effect
+        assert wide < 10 * tight
