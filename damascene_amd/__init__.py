@@ -298,6 +298,13 @@ class Context:
         check(lib().dmsc_eigensolve_report(self.handle, ctypes.byref(rule), ctypes.byref(res)))
         return rule.value, res.value
 
+    def resident_report(self):
+        """dmsc_resident_report: (launches with waiting blocks run to their
+        end, given up) by this context's solves so far."""
+        done, stalled = ctypes.c_int(), ctypes.c_int()
+        check(lib().dmsc_resident_report(self.handle, ctypes.byref(done), ctypes.byref(stalled)))
+        return done.value, stalled.value
+
     def spectral_pb(self, eigvals, eigvecs):
         nvec, h, w = eigvecs.shape
         pitch = pitch_in_floats(w * h)

@@ -511,6 +511,18 @@ int dmsc_eigensolve_report(dmsc_ctx* ctx, int* stop_rule, double* max_residual) 
   return DMSC_OK;
 }
 
+int dmsc_resident_report(dmsc_ctx* ctx, int* completed, int* stalled) {
+  CHECK_CTX(ctx);
+  DMSC_ARG(completed && stalled, "null pointer");
+  *completed = ctx->resident_completed;
+  *stalled = ctx->resident_stalled;
+  for (const Ctx* lane : ctx->lanes) {
+    *completed += lane->resident_completed;
+    *stalled += lane->resident_stalled;
+  }
+  return DMSC_OK;
+}
+
 int dmsc_find_textons(dmsc_ctx* ctx, int w, int h, const float* grey, int* textons, int texton_choice,
                       int precision, int* iterations) {
   CHECK_CTX(ctx);

@@ -1281,11 +1281,13 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
     // iteration, read here)
     DMSC_HIP(hipStreamSynchronize(s));
     if (whole && *h_stalled) {  // the grid was not resident in time: this iteration again, one launch per step
+      ctx->resident_stalled++;
       whole = false;
       gate.reset();
       outer--;
       continue;
     }
+    if (whole) ctx->resident_completed++;
     const auto t_rr = std::chrono::steady_clock::now();
     if (!rayleigh_ritz(h_gram, h_gram + kB * kB, kB, theta, S))
       return fail(DMSC_ERR_INTERNAL, "block eigensolver: filtered block lost rank at outer iteration %d", outer);

@@ -44,6 +44,8 @@ struct Ctx {
   // largest residual |A u - lambda u| of its wanted pairs at that point
   int eig_stop = 0;
   double eig_residual = 0.0;
+  // resident launches of this context's solves: run to their end, given up
+  int resident_completed = 0, resident_stalled = 0;
   ~Ctx();
   int pinned(int** out);
   int aux_stream(hipStream_t* s, hipEvent_t* ev0, hipEvent_t* ev1);

@@ -1787,6 +1787,7 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
         DMSC_HIP(hipStreamSynchronize(s));
       }
       if (hs.stalled) {  // the grid was not resident in time: the same solve with two kernels per step
+        ctx->resident_stalled++;
         gate.reset();
         return solve(ctx, w, h, A, pitch, nvec, tol, mixed, h_eigvals, d_eigvecs, iterations, 0, nullptr, force, false,
                      false);
@@ -1809,6 +1810,7 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
         return fail(DMSC_ERR_NOCONV, "Cullum screening kept %d of %d values at m=%d with %d candidates",
                     hs.nscreened, nvec, done, ncheck);
     }
+    if (resident) ctx->resident_completed++;
     if (hs.fail == 2) return fail(DMSC_ERR_INTERNAL, "inverse iteration failed on the Lanczos tridiagonal");
     if (hs.fail == 0) {
       bool good = true;  // lanczos.cu:114-140 TestForConvergence

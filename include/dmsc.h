@@ -201,6 +201,11 @@ int dmsc_generalized_eigensolve(dmsc_ctx* ctx, int w, int h, float* d_matrix, in
  *                       last check's Ritz pairs (lanczos.cu:519-560). */
 enum { DMSC_STOP_NONE = 0, DMSC_STOP_RESIDUAL = 1, DMSC_STOP_STEADY = 2, DMSC_STOP_FLOOR = 3, DMSC_STOP_CAP = 4 };
 int dmsc_eigensolve_report(dmsc_ctx* ctx, int* stop_rule, double* max_residual);
+/* No reference counterpart: the launches with blocks that wait for each other
+ * (the "resident_polls" tuning value) that this context's solves and its batch
+ * lanes' have run since it was made: to their end, and given up because a wait
+ * ran out of polls (their work was done again with launches per step). */
+int dmsc_resident_report(dmsc_ctx* ctx, int* completed, int* stalled);
 /* spectralPb.h:19 spectralPb -> [8][pitch] (accumulates into d_spb after
  * zeroing it). */
 int dmsc_spectral_pb(dmsc_ctx* ctx, const float* h_eigvals, const float* d_eigvecs, int w,
