@@ -335,7 +335,8 @@ def pmc_workload(shape):
     torch.cuda.synchronize()
     m3 = ctx.intervene(out["nmax"])
     ctx.convert_matrix(W, H, m3)
-    check(lib().dmsc_chebyshev_time_products(ctx.handle, W, H, m3.data_ptr(), m3.shape[1], 50, ctypes.byref(ms)))
+    with dm.tuned(resident_polls=0):  # one launch per step
+        check(lib().dmsc_chebyshev_time_products(ctx.handle, W, H, m3.data_ptr(), m3.shape[1], 50, ctypes.byref(ms)))
     torch.cuda.synchronize()
     d_rgb = ctx.upload(dm.generate_image(W, H, CELLS, SEED))
     resp = ctx.texton_responses(ctx.rgb_to_grey(d_rgb))
@@ -371,13 +372,15 @@ def filter_roofline(ctx, nmax):
     tile, HIP events on the library's stream over FILTER_TIMED launches on
     the image's L_sym) and its roofline: HBM on 708 algorithmic bytes per
     row, with its FP32 multiply-adds against the FP32 peak beside it."""
+    import damascene_amd as dm
     from damascene_amd._lib import check, lib
 
     m = ctx.intervene(nmax)
     ctx.convert_matrix(W, H, m)
     ms = ctypes.c_float()
-    check(lib().dmsc_chebyshev_time_products(ctx.handle, W, H, m.data_ptr(), m.shape[1], FILTER_TIMED,
-                                             ctypes.byref(ms)))
+    with dm.tuned(resident_polls=0):  # one launch per step
+        check(lib().dmsc_chebyshev_time_products(ctx.handle, W, H, m.data_ptr(), m.shape[1], FILTER_TIMED,
+                                                 ctypes.byref(ms)))
     tile = ctx.chebyshev_tile(W, H)
     kernel = FILTER_KERNELS.get(tile, f"filter tile {tile}")
     avg_s = ms.value / 1e3

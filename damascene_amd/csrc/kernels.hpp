@@ -151,10 +151,13 @@ void release_local_cues(const Ctx* ctx);   // drops the context's cached local-c
 int time_lanczos_steps(Ctx* ctx, int w, int h, float* A, int pitch, int precision, int steps, float* ms_per_step);
 // Step-kernel shape of the Lanczos solver: mixed step form (0 two kernels,
 // 1 linear fused, 2 tiled fused), tile code (width * 100 + height) and
-// block size (0 = default); ms is the measured time per step.
+// block size (0 = default); ms is the measured time per step; resident: plain
+// steps run in one launch per check period where that serves the size (and k1
+// is 0 or 256).
 struct StepShape {
   int fused, tile, k1;
   float ms;
+  bool resident;
 };
 // Tiles of the tiled fused mixed step (width * 100 + height); the first is
 // the default.

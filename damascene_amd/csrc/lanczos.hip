@@ -1476,7 +1476,7 @@ StepShape default_shape(int w, int h, bool mixed) {
     auto it = tuned_shapes().find(std::make_tuple(w, h, mixed ? 1 : 0));
     if (it != tuned_shapes().end()) return it->second;
   }
-  return StepShape{mixed ? lanczos_mixed_fused : 0, lanczos_tile, lanczos_k1_threads, 0.f};
+  return StepShape{mixed ? lanczos_mixed_fused : 0, lanczos_tile, lanczos_k1_threads, 0.f, true};
 }
 
 // time_steps > 0: run that many steps with no checks between two HIP
@@ -1484,8 +1484,10 @@ StepShape default_shape(int w, int h, bool mixed) {
 // *ms_per_step (the measurement mode of dmsc_lanczos_time_steps).  `force`
 // selects the step-kernel shape (the autotuner's trials); otherwise the
 // autotuned shape of this size, else the process-wide tuning values.
-// run == false: never k_lz_run.  convert == false: A already holds L_sym (a later timing run on the same
-// matrix).
+// run == false: never k_lz_run.  convert == false: A already holds L_sym (a
+// later timing run on the same matrix).  A timing run whose `force` wants
+// k_lz_run times that alone: 0 ms if the size is not served, -1 if it could not
+// be timed now.
 int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool mixed, float* h_eigvals,
           float* d_eigvecs, int* iterations, int time_steps = 0, float* ms_per_step = nullptr,
           const StepShape* force = nullptr, bool convert = true, bool run = true) {
@@ -1640,7 +1642,41 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
   }
   DMSC_HIP(hipGetLastError());
 
+  // Plain steps in one resident launch per check period where the grid fits
+  // the device (262,144 rows on 256 compute units) and no other resident
+  // launch runs on it; 500 steps with their check take 3.3 ms against 5.9
+  // at 61x37, 3.6 against 7.4 at 481x321, 4.7 against 10.2 at 512x512 and,
+  // with the widest halo, 7.5 against 9.5 at 3000x80.
+  // Beside other kernels it holds its own: six images over four batch lanes
+  // take 33 ms with it, 38 ms with two kernels per step.
+  std::unique_ptr<ResidentGrid> gate;
+  bool served = false, resident = false;
+  unsigned long long* slots = (unsigned long long*)(B + o_slots);
+  if (!mixed) {
+    if (k1 == kRed && shape.resident && run && resident_polls > 0)
+      DMSC_TRY(run_fits(ctx->device, n, p.so, w, &served));
+    if (served) gate = std::make_unique<ResidentGrid>(ctx->device);
+    resident = served && gate->held();
+  }
+  const auto enqueue = [&](int first, int steps) -> int {
+    if (resident) {
+      hipLaunchKernelGGL(k_lz_slots, dim3(div_up(std::max(4 * slot_stride, n), 256)), dim3(256), 0, s, slots,
+                         4 * slot_stride, (unsigned*)((first & 1) ? p.plain.z1 : p.plain.z0), n);
+      hipLaunchKernelGGL(k_lz_run, dim3(div_up(n, kRunRows)), dim3(kRunRows), run_lds(p.so.halo), s, p.plain, w,
+                         p.so.halo, first, steps, slots, slot_stride, resident_polls);
+      DMSC_HIP(hipGetLastError());
+      return DMSC_OK;
+    }
+    for (int t = 0; t < steps; t += kGraphSteps)
+      DMSC_TRY(run_steps(ctx, p, st, w, first + t, std::min(kGraphSteps, steps - t)));
+    return DMSC_OK;
+  };
+
   if (time_steps > 0) {
+    if (force && force->resident && !resident) {  // a trial of the launch alone
+      *ms_per_step = served ? -1.f : 0.f;
+      return DMSC_OK;
+    }
     const int steps = std::min(time_steps, kMaxIter - kGraphSteps);
     if ((size_t)steps + kGraphSteps + 2 > cap) {
       void* nbuf;
@@ -1653,13 +1689,12 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
       hipLaunchKernelGGL(k_set_basis, dim3(1), dim3(1), 0, s, st, V);
     }
     // steps 0..24 build the graph and warm up; steps 25.. are timed
-    DMSC_TRY(run_steps(ctx, p, st, w, 0, kGraphSteps));
+    DMSC_TRY(enqueue(0, kGraphSteps));
     hipEvent_t e0, e1;
     DMSC_HIP(hipEventCreate(&e0));
     DMSC_HIP(hipEventCreate(&e1));
     DMSC_HIP(hipEventRecord(e0, s));
-    for (int t = 0; t < steps; t += kGraphSteps)
-      DMSC_TRY(run_steps(ctx, p, st, w, kGraphSteps + t, std::min(kGraphSteps, steps - t)));
+    DMSC_TRY(enqueue(kGraphSteps, steps));
     DMSC_HIP(hipEventRecord(e1, s));
     DMSC_HIP(hipEventSynchronize(e1));
     float ms = 0;
@@ -1667,23 +1702,22 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     *ms_per_step = ms / (float)steps;
+    if (resident) {
+      int stalled = 0;
+      DMSC_HIP(hipMemcpyAsync(&stalled, &st->stalled, sizeof(int), hipMemcpyDeviceToHost, s));
+      DMSC_HIP(hipStreamSynchronize(s));
+      if (!stalled) {
+        ctx->resident_completed += 2;
+      } else {
+        ctx->resident_stalled++;
+        gate.reset();
+        if (!force)
+          return solve(ctx, w, h, A, pitch, nvec, tol, mixed, nullptr, nullptr, nullptr, time_steps, ms_per_step,
+                       nullptr, false, false);
+        *ms_per_step = -1.f;
+      }
+    }
     return DMSC_OK;
-  }
-
-  // Plain steps in one resident launch per check period where the grid fits
-  // the device (262,144 rows on 256 compute units) and no other resident
-  // launch runs on it; 500 steps with their check take 3.3 ms against 5.9
-  // at 61x37, 3.6 against 7.4 at 481x321, 4.7 against 10.2 at 512x512 and,
-  // with the widest halo, 7.5 against 9.5 at 3000x80.
-  // Beside other kernels it holds its own: six images over four batch lanes
-  // take 33 ms with it, 38 ms with two kernels per step.
-  std::unique_ptr<ResidentGrid> gate;
-  bool resident = false;
-  unsigned long long* slots = (unsigned long long*)(B + o_slots);
-  if (!mixed) {
-    if (k1 == kRed && run && resident_polls > 0) DMSC_TRY(run_fits(ctx->device, n, p.so, w, &resident));
-    if (resident) gate = std::make_unique<ResidentGrid>(ctx->device);
-    resident = resident && gate->held();
   }
 
   int eigCheck = nvec + kCullumExtra;
@@ -1730,16 +1764,7 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
       cap = ncap;
       hipLaunchKernelGGL(k_set_basis, dim3(1), dim3(1), 0, s, st, V);
     }
-    if (resident) {
-      hipLaunchKernelGGL(k_lz_slots, dim3(div_up(std::max(4 * slot_stride, n), 256)), dim3(256), 0, s, slots,
-                         4 * slot_stride, (unsigned*)((done & 1) ? p.plain.z1 : p.plain.z0), n);
-      hipLaunchKernelGGL(k_lz_run, dim3(div_up(n, kRunRows)), dim3(kRunRows), run_lds(p.so.halo), s, p.plain, w,
-                         p.so.halo, done, steps, slots, slot_stride, resident_polls);
-      DMSC_HIP(hipGetLastError());
-    } else {
-      for (int t = ahead; t < steps; t += kGraphSteps)
-        DMSC_TRY(run_steps(ctx, p, st, w, done + t, std::min(kGraphSteps, steps - t)));
-    }
+    DMSC_TRY(enqueue(done + ahead, steps - ahead));
     done += steps;
     ahead = 0;
     if (mixed) {
@@ -1864,7 +1889,8 @@ int time_lanczos_steps(Ctx* ctx, int w, int h, float* A, int pitch, int precisio
 
 // Times every step-kernel shape for this size and precision (25 warm-up
 // and `steps` timed steps each, on the matrix converted once in place),
-// records the fastest as the size's shape and returns every trial.
+// returns every trial and records the fastest as the size's shape, or, for
+// plain steps, the launch of a whole check period where that is faster still.
 int autotune_steps(Ctx* ctx, int w, int h, float* A, int pitch, int precision, int steps, StepShape* best,
                    StepShape* tried, int max_tried, int* n_tried) {
   if (pitch % 4) return fail(DMSC_ERR_ARG, "matrix pitch must be a multiple of 4 floats");
@@ -1873,26 +1899,39 @@ int autotune_steps(Ctx* ctx, int w, int h, float* A, int pitch, int precision, i
   const bool mixed = precision == DMSC_PREC_MIXED;
   std::vector<StepShape> cand;
   if (mixed) {
-    for (int tile : kStepTiles) cand.push_back(StepShape{2, tile, 0, 0.f});
-    for (int k1 : {512, 256}) cand.push_back(StepShape{1, 0, k1, 0.f});
-    for (int k1 : {256, 64}) cand.push_back(StepShape{0, 0, k1, 0.f});
+    for (int tile : kStepTiles) cand.push_back(StepShape{2, tile, 0, 0.f, false});
+    for (int k1 : {512, 256}) cand.push_back(StepShape{1, 0, k1, 0.f, false});
+    for (int k1 : {256, 64}) cand.push_back(StepShape{0, 0, k1, 0.f, false});
   } else {
-    for (int k1 : {256, 64}) cand.push_back(StepShape{0, 0, k1, 0.f});
+    for (int k1 : {256, 64}) cand.push_back(StepShape{0, 0, k1, 0.f, false});
   }
   int nt = 0;
   StepShape top{};
   top.ms = 0.f;
+  const auto trial = [&](const StepShape& c, bool convert, float* ms) {
+    return solve(ctx, w, h, A, pitch, 9, 1e-3f, mixed, nullptr, nullptr, nullptr, steps, ms, &c, convert);
+  };
   for (StepShape c : cand) {
     float ms = 0.f;
-    DMSC_TRY(solve(ctx, w, h, A, pitch, 9, 1e-3f, mixed, nullptr, nullptr, nullptr, steps, &ms, &c, nt == 0));
+    DMSC_TRY(trial(c, nt == 0, &ms));
     c.ms = ms;
     if (tried && nt < max_tried) tried[nt] = c;
     nt++;
     if (top.ms == 0.f || ms < top.ms) top = c;
   }
+  StepShape keep = top;
+  if (!mixed) {
+    // k_lz_run against the fastest pair of kernels: a served size keeps it
+    // unless it was timed and slower.  Beside it, for solves that may not take
+    // it, go the kernels that give the same bits (256 rows).
+    const StepShape run{0, 0, kRed, 0.f, true};
+    float ms = 0.f;
+    DMSC_TRY(trial(run, false, &ms));
+    if (ms < 0.f || (ms > 0.f && ms <= top.ms)) keep = run;
+  }
   {
     std::lock_guard<std::mutex> lk(tuned_lock());
-    tuned_shapes()[std::make_tuple(w, h, mixed ? 1 : 0)] = top;
+    tuned_shapes()[std::make_tuple(w, h, mixed ? 1 : 0)] = keep;
   }
   if (best) *best = top;
   if (n_tried) *n_tried = nt;

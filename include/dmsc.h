@@ -241,7 +241,8 @@ int dmsc_write_pgm(const char* path, int w, int h, const float* h_data);
  *   "lanczos_k1_threads": rows per block of the eigensolver's SpMV step
  *                         kernel: 0 = automatic (default: 256 for two-kernel
  *                         steps, 512 for the fused mixed step), 64, 256 or
- *                         512 (512 applies to the fused step only).
+ *                         512 (512 applies to the fused step only).  At 64
+ *                         plain solves take two kernels per step at any size.
  *   "resident_polls":     the launches whose blocks wait for each other (a
  *                         check period of the plain eigensolver, an outer
  *                         iteration's filter of the block eigensolver): how
@@ -271,10 +272,11 @@ int dmsc_write_pgm(const char* path, int w, int h, const float* h_data);
  *   "lanczos_trace":      non-zero prints one line per eigensolver check to
  *                         stderr (2: also the Ritz values of a failed
  *                         screening).
- *   "eigensolver":        mixed precision only: 0 Lanczos (the default), 1
+ *   "eigensolver":        mixed precision only: 0 Lanczos, 1 (the default)
  *                         Chebyshev-filtered subspace iteration on a block of
  *                         32 vectors with an FP64 Rayleigh-Ritz step (no
- *                         reference counterpart; nvec <= 16).  It stops when
+ *                         reference counterpart; nvec <= 16, more take
+ *                         Lanczos).  It stops when
  *                         every wanted residual is at most
  *                         tol * 10^-lanczos_mixed_stop, when no wanted Ritz
  *                         vector moved by more than 0.03 tol (sine of the
@@ -283,9 +285,15 @@ int dmsc_write_pgm(const char* path, int w, int h, const float* h_data);
  *                         (dmsc_eigensolve_report tells which); the iteration
  *                         count it reports is the number of block products
  *                         with the matrix.
- *   "chebyshev_shape":    its filter kernel's tile, rows per lane * 10 +
- *                         float4 planes per lane: 24 (the default), 28, 22
- *                         or 42.
+ *   "chebyshev_shape":    its filter kernel's tile: 0 (the default) = chosen
+ *                         by size (dmsc_chebyshev_tile), and one launch per
+ *                         outer iteration where that serves the size; else
+ *                         always one launch per step with rows per lane * 10 +
+ *                         float4 planes per lane (24, 28, 22, 42), or 300 +
+ *                         rows * 10 + waves on LDS tiles (324, 328, 342, 344,
+ *                         348; + 1000 with pipelined matrix loads: 1324, 1328,
+ *                         1336, 1337, 1344, 1348; + 2000 with LDS read-ahead:
+ *                         2324, 2328, 2337).
  *   "overlap_stages":     dmsc_gpb runs the L, a and b local cues on the
  *                         context's second stream beside the textons (1, the
  *                         default) or every stage in order on one stream (0;
@@ -297,18 +305,23 @@ int dmsc_write_pgm(const char* path, int w, int h, const float* h_data);
  * `steps` (a multiple of 25) Lanczos steps of the given precision with no
  * convergence checks between two HIP events on the context's stream, after
  * 25 untimed steps, and returns the average milliseconds per step.  The step
- * kernels are the ones dmsc_generalized_eigensolve uses. */
+ * kernels are the ones dmsc_generalized_eigensolve uses: plain steps of sizes
+ * that take one launch per check period run in such launches. */
 int dmsc_lanczos_time_steps(dmsc_ctx* ctx, int w, int h, float* d_matrix, int matrix_pitch, int precision,
                             int steps, float* ms_per_step);
 /* No reference counterpart: times `products` filter steps of the block
  * eigensolver (eigensolver = 1) on a converted matrix (L_sym, as
- * dmsc_convert_matrix leaves it) with the tile dmsc_chebyshev_tile names, a
- * block of 32 vectors, after 5 untimed steps, with HIP events on the
- * context's stream; returns the average milliseconds per step. */
+ * dmsc_convert_matrix leaves it), a block of 32 vectors, with HIP events on the
+ * context's stream, as a block solve of this size runs them: in launches of up
+ * to 300 steps where it takes those (after an untimed one), else one launch per
+ * step with the tile dmsc_chebyshev_tile names (after 5 untimed ones).  Returns
+ * the average milliseconds per step. */
 int dmsc_chebyshev_time_products(dmsc_ctx* ctx, int w, int h, const float* d_matrix, int matrix_pitch,
                                  int products, float* ms_per_product);
 /* No reference counterpart: the filter tile (a chebyshev_shape value) that a
- * block solve at w x h uses on this context's device: the autotuner's pick
+ * block solve at w x h uses on this context's device (for the products outside
+ * the filter too; at sizes whose filter runs in one launch per outer iteration,
+ * for those alone): the autotuner's pick
  * for that size, else the tuning key, else (key 0, the default) 2337 where
  * its grid fits in one round of the device's block slots and 2328's does
  * not, else 2328. */
@@ -316,9 +329,11 @@ int dmsc_chebyshev_tile(dmsc_ctx* ctx, int w, int h, int* shape);
 /* No reference counterpart: times every filter tile of the block eigensolver
  * (the 18 chebyshev_shape values) at w x h on a converted matrix, `products`
  * steps each, and makes the fastest the tile of later block solves at that
- * size (tiles give bit-identical results).  shapes_tried/us_per_product
- * receive up to max_tried (tile, microseconds per step) pairs;
- * dmsc_autotune_clear forgets the choices. */
+ * size (tiles give bit-identical results).  Where the filter can run in one
+ * launch per outer iteration that form is timed too, and later solves keep it
+ * unless the fastest tile beats it by more than 3 %.
+ * shapes_tried/us_per_product receive up to max_tried (tile, microseconds per
+ * step) pairs; dmsc_autotune_clear forgets the choices. */
 int dmsc_autotune_chebyshev(dmsc_ctx* ctx, int w, int h, const float* d_matrix, int matrix_pitch, int products,
                             int* best_shape, int* shapes_tried, float* us_per_product, int max_tried,
                             int* n_tried);
@@ -330,9 +345,13 @@ int dmsc_autotune_chebyshev(dmsc_ctx* ctx, int w, int h, const float* d_matrix, 
  * of 512 and 256 rows per block, two-kernel steps of 256 and 64; plain:
  * two-kernel steps of 256 and 64 -- with `steps` (a multiple of 25) timed
  * steps each, and records the fastest as the shape every later eigensolve
- * of this size and precision uses (in this process).  Shapes change results
- * only through the rounding of block partial sums.  `tried` receives up to
- * max_tried trials, *n_tried their number. */
+ * of this size and precision uses (in this process).  Plain steps of sizes
+ * that can run in one launch per check period are timed in that form too, and
+ * where it is the fastest later solves keep it, and the 256-row kernels with
+ * the same results where it cannot be had; `best` is then the fastest of the
+ * two-kernel shapes.  Shapes change results only through the rounding of block
+ * partial sums.  `tried` receives up to max_tried trials, *n_tried their
+ * number. */
 typedef struct {
   int mixed_fused;    /* 0 two kernels, 1 linear fused, 2 tiled fused (mixed only) */
   int tile;           /* tiled step: tile width * 100 + height */

@@ -1,10 +1,13 @@
 """Which solves run in launches whose blocks wait for each other: the results
 are the same either way, so the context's report tells."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import damascene_amd as dm
+from damascene_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +84,68 @@ def test_batch_report(own):
     torch.cuda.synchronize()
     done, stalled = own.resident_report()
     assert done > 0 and stalled == 0 and len(out) == 4
+
+
+@pytest.fixture
+def untuned():
+    check(lib().dmsc_autotune_clear())
+    yield
+    check(lib().dmsc_autotune_clear())
+
+
+# a tuned size keeps the launch, whichever of the two-kernel shapes was the
+# faster one, and with it the results
+@pytest.mark.parametrize("w,h", [(32, 32), (64, 48), (160, 120), (230, 57), (481, 321)])
+def test_tuned_plain_size_keeps_the_launch(own, untuned, w, h):
+    with dm.tuned(resident_polls=ALWAYS):
+        before, _ = solve(own, w, h, dm.PREC_FP32)
+        m = own.intervene(torch.rand(h, w, device="cuda"))
+        best, trials = own.autotune_eigensolver(w, h, m, precision=dm.PREC_FP32, steps=200)
+        print(f"case: tuned {w}x{h}: best {best}", flush=True)
+        after, (done, stalled) = solve(own, w, h, dm.PREC_FP32)
+    assert done > 0 and stalled == 0 and after == before
+
+
+def product_us(c, w, h, m, products=100):
+    ms = ctypes.c_float()
+    check(lib().dmsc_chebyshev_time_products(c.handle, w, h, m.data_ptr(), m.shape[1], products, ctypes.byref(ms)))
+    return ms.value * 1e3
+
+
+# the block filter's trials decide between the launch and the fastest tile: at
+# wide tiles with few columns in use the tile may win
+@pytest.mark.parametrize("w,h", [(320, 240), (481, 321), (33, 2100), (64, 1200)])
+def test_tuned_filter_takes_the_faster_form(own, untuned, w, h):
+    with dm.tuned(resident_polls=ALWAYS):
+        before, _ = solve(own, w, h, dm.PREC_MIXED)
+        m = own.intervene(torch.rand(h, w, device="cuda"))
+        own.convert_matrix(w, h, m)
+        count = own.resident_report()[0]
+        launch = min(product_us(own, w, h, m) for _ in range(3))
+        served = own.resident_report()[0] > count
+        best, us = own.autotune_chebyshev(w, h, m, products=100)
+        after, (done, stalled) = solve(own, w, h, dm.PREC_MIXED)
+    print(f"case: filter {w}x{h}: launch {launch:.1f} us ({served}), tile {best} {us[best]:.1f} us, taken {done}",
+          flush=True)
+    assert served and stalled == 0 and after == before
+    if launch < 0.8 * us[best]:
+        assert done > 0
+    if us[best] < 0.8 * launch:
+        assert done == 0
+
+
+# the measuring entry points run what a solve of the size runs
+def test_timed_steps_are_the_solves(own, untuned):
+    print("case: timed steps", flush=True)
+    w, h = 481, 321
+    ms = ctypes.c_float()
+    for polls, launches in ((ALWAYS, True), (0, False)):
+        with dm.tuned(resident_polls=polls):
+            a = own.resident_report()[0]
+            m = own.intervene(torch.rand(h, w, device="cuda"))
+            check(lib().dmsc_lanczos_time_steps(own.handle, w, h, m.data_ptr(), m.shape[1], dm.PREC_FP32, 200,
+                                                ctypes.byref(ms)))
+            b = own.resident_report()[0]
+            product_us(own, w, h, m)
+            c = own.resident_report()[0]
+        assert ms.value > 0 and (b > a) == launches and (c > b) == launches
