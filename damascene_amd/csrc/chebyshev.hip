@@ -1250,7 +1250,7 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
   RunShape rs;
   if (run_wanted(w, h)) DMSC_TRY(run_shape(ctx->device, w, h, &rs));
   std::unique_ptr<ResidentGrid> gate;
-  if (rs.units) gate = std::make_unique<ResidentGrid>(ctx->device);
+  if (rs.units && ctx->resident_backoff.due(resident_polls)) gate = std::make_unique<ResidentGrid>(ctx->device);
   bool whole = gate && gate->held();
   int* stalled = (int*)(Bp + o_stall);
   int* h_stalled = (int*)(h_gram + (size_t)kGrams * kB * kB);
@@ -1296,12 +1296,16 @@ int chebyshev_solve(Ctx* ctx, int w, int h, const float* A, int pitch, int nvec,
     DMSC_HIP(hipStreamSynchronize(s));
     if (whole && *h_stalled) {  // the grid was not resident in time: this iteration again, one launch per step
       ctx->resident_stalled++;
+      ctx->resident_backoff.stalled(resident_polls);
       whole = false;
       gate.reset();
       outer--;
       continue;
     }
-    if (whole) ctx->resident_completed++;
+    if (whole) {
+      ctx->resident_completed++;
+      ctx->resident_backoff.completed();
+    }
     const auto t_rr = std::chrono::steady_clock::now();
     if (!rayleigh_ritz(h_gram, h_gram + kB * kB, kB, theta, S))
       return fail(DMSC_ERR_INTERNAL, "block eigensolver: filtered block lost rank at outer iteration %d", outer);

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "dmsc.h"
+#include "resident_gate.hpp"
 #include "tables.hpp"
 
 namespace dmsc {
@@ -46,6 +47,7 @@ struct Ctx {
   double eig_residual = 0.0;
   // resident launches of this context's solves: run to their end, given up
   int resident_completed = 0, resident_stalled = 0;
+  ResidentBackoff resident_backoff;
   ~Ctx();
   int pinned(int** out);
   int aux_stream(hipStream_t* s, hipEvent_t* ev0, hipEvent_t* ev1);

@@ -1655,8 +1655,10 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
   if (!mixed) {
     if (k1 == kRed && shape.resident && run && resident_polls > 0)
       DMSC_TRY(run_fits(ctx->device, n, p.so, w, &served));
-    if (served) gate = std::make_unique<ResidentGrid>(ctx->device);
-    resident = served && gate->held();
+    // (a timing run wants it whatever happened to the solves before)
+    if (served && (time_steps > 0 || ctx->resident_backoff.due(resident_polls)))
+      gate = std::make_unique<ResidentGrid>(ctx->device);
+    resident = gate && gate->held();
   }
   const auto enqueue = [&](int first, int steps) -> int {
     if (resident) {
@@ -1813,6 +1815,7 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
       }
       if (hs.stalled) {  // the grid was not resident in time: the same solve with two kernels per step
         ctx->resident_stalled++;
+        ctx->resident_backoff.stalled(resident_polls);
         gate.reset();
         return solve(ctx, w, h, A, pitch, nvec, tol, mixed, h_eigvals, d_eigvecs, iterations, 0, nullptr, force, false,
                      false);
@@ -1835,7 +1838,10 @@ int solve(Ctx* ctx, int w, int h, float* A, int pitch, int nvec, float tol, bool
         return fail(DMSC_ERR_NOCONV, "Cullum screening kept %d of %d values at m=%d with %d candidates",
                     hs.nscreened, nvec, done, ncheck);
     }
-    if (resident) ctx->resident_completed++;
+    if (resident) {
+      ctx->resident_completed++;
+      ctx->resident_backoff.completed();
+    }
     if (hs.fail == 2) return fail(DMSC_ERR_INTERNAL, "inverse iteration failed on the Lanczos tridiagonal");
     if (hs.fail == 0) {
       bool good = true;  // lanczos.cu:114-140 TestForConvergence

@@ -39,4 +39,29 @@ class ResidentGrid {
   bool held_ = false;
 };
 
+// After a launch has given up (another process holds compute units it waits
+// for) a context's next solves do without: one, then two, four, ... up to 64
+// between two attempts, until a launch runs to its end again.  So a device that
+// stays shared costs few waits, each as long as the poll bound lets it be.  A
+// larger bound than the one that ran out is tried at once.
+class ResidentBackoff {
+ public:
+  // Whether a solve that could take the launch should.
+  bool due(int polls) {
+    if (skip_ == 0 || polls > polls_) return true;
+    skip_--;
+    return false;
+  }
+  void stalled(int polls) {
+    polls_ = polls;
+    wait_ = wait_ == 0 ? 1 : wait_ < kMost ? 2 * wait_ : kMost;
+    skip_ = wait_;
+  }
+  void completed() { wait_ = skip_ = 0; }
+
+ private:
+  static constexpr int kMost = 64;
+  int polls_ = 0, wait_ = 0, skip_ = 0;
+};
+
 }  // namespace dmsc

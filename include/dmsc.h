@@ -248,8 +248,11 @@ int dmsc_write_pgm(const char* path, int w, int h, const float* h_data);
  *                         iteration's filter of the block eigensolver): how
  *                         often a block looks for another's value before the
  *                         work is done again with launches per step (0-2^20,
- *                         16384; 0 = always launches per step, for a GPU that
- *                         several processes share; results are identical).
+ *                         16384; 0 = always launches per step; results are
+ *                         identical).  After such a wait has run out (a GPU
+ *                         that other processes keep busy) the context's next
+ *                         solves keep to launches per step, one, then two,
+ *                         four, ... up to 64 of them between two attempts.
  *   "lanczos_mixed_fused": mixed eigensolver step as one kernel staging the
  *                         basis vector in LDS, over pixel tiles (2, default)
  *                         or runs of consecutive rows (1, when the stencil

@@ -75,6 +75,22 @@ def test_given_up_and_taken_again(own, w, h, precision):
     assert done > 0 and stalled == 0 and first == second
 
 
+# a device that stays busy: after a launch has given up the next solves do
+# without, one, then two
+@pytest.mark.parametrize("w,h,precision", [(230, 57, dm.PREC_FP32), (320, 240, dm.PREC_MIXED)])
+def test_given_up_is_remembered(own, w, h, precision):
+    print(f"case: remembered {w}x{h} precision {precision}", flush=True)
+    with dm.tuned(resident_polls=1):
+        tries = [solve(own, w, h, precision) for _ in range(6)]
+        print([t[1] for t in tries], flush=True)
+    assert all(t[0] == tries[0][0] for t in tries)
+    stalled = [t[1][1] for t in tries]
+    assert precision == dm.PREC_MIXED or sum(stalled) > 0  # a thousand waits or more of one poll each
+    for i, t in enumerate(tries[:-1]):
+        if t[1][1]:
+            assert tries[i + 1][1] == (0, 0)
+
+
 # a batch: the lanes' launches are in the report, and one lane at a time has them
 def test_batch_report(own):
     print("case: resident launches of a batch", flush=True)
