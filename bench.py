@@ -3,8 +3,8 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--no-batch]
 
 A step is one full gPb pass (RGB8 resident in HBM -> oriented gPb) over one
-481x321 image.  `value` is images/s of the mixed-precision path: BF16 MFMA
-k-means distances with an exact FP32 re-check, and the block eigensolver
+481x321 image.  `value` is images/s of the mixed-precision path: exact FP32 k-means
+distances on the matrix cores (as the plain path's), and the block eigensolver
 (Chebyshev-filtered subspace iteration on 32 FP32 vectors, FP64 Gram
 matrices, Rayleigh-Ritz and residuals).  The plain FP32 path (the reference
 algorithm) and the mixed path on its Lanczos solver are timed beside it, and
@@ -13,20 +13,18 @@ tests/golden/truth_481x321.npz (eigenvalue relative error, subspace angle of
 eigenvectors 1..8, gPb max-abs error, nonmax mismatches against the oracle).
 
 roofline: the dominant work of the timed region, the block solver's filter
-step, in its form of one launch per step at the tile the library picks at
-481x321 (reported as `tile`: 2337, k_cheb_ldp<3, 7>, 64 x 21 pixels per block,
-whose 512 blocks fill one round of the chip's block slots).  The timed solve
-itself runs all steps of an outer iteration in one launch at this size
-(k_cheb_run), faster than these figures.  One launch per filter step
-forms the 81-diagonal stencil product of a block of 32 vectors, y = a (A x -
-c x) - b z, at 708 algorithmic bytes per row (the matrix row 324 B; x, z and
-y 128 B each).  Its average duration is measured with HIP events on the
-library's stream over
-FILTER_TIMED launches; `traffic` is the HBM bytes per launch from the
-rocprofv3 FETCH_SIZE/WRITE_SIZE runs committed under profiles/.  Beside it:
-`valu` (the same launch's FP32 multiply-adds against the FP32 peak),
-`lanczos_step` (the fused mixed Lanczos step, 348 B per row) and `spmv` (the
-standalone SpMV, 332 B per row, over its launch shapes).
+step, y = a (A x - c x) - b z with the 81-diagonal stencil product of a block of
+32 vectors, as the timed solve runs it at 481x321: all steps of an outer
+iteration in one launch (k_cheb_run), whose blocks keep the matrix in registers
+and exchange only tile frames, so it is priced by its FP32 multiply-adds (5,184
+flop per row) against the FP32 matrix peak.  The average time per step is
+measured with HIP events on the library's stream over FILTER_TIMED steps;
+`traffic` is the HBM bytes per step from the rocprofv3 FETCH_SIZE/WRITE_SIZE
+runs committed under profiles/.  Beside it: `launch_per_step` (the same step as
+one launch, the form of other sizes, at the tile the library picks at 481x321,
+against HBM on 708 algorithmic bytes per row: the matrix row 324 B; x, z and y
+128 B each), `lanczos_step` (the fused mixed Lanczos step, 348 B per row) and
+`spmv` (the standalone SpMV, 332 B per row, over its launch shapes).
 
 batched: dmsc_gpb_batch over 16 images of 481x321 (seeds 20261202 + i) and
 over 64 images of uneven size (sides uniform in [200, 1024]), 4 concurrent
@@ -67,10 +65,12 @@ SPMV_SHAPES = {0: "k_spmv_full", 1: "k_spmv<1>", 2: "k_spmv<2>", 4: "k_spmv<4>"}
 STEP_KERNEL = "k_lzmt<32, 8, 0>"
 STEP_BYTES_PER_ROW = 81 * 4 + 8 + 4 + 4 + 8
 STEP_TIMED = 500
-# block eigensolver filter step (the default tile), per row: the matrix row
-# (324 B) and, for 32 vectors, x, z read and y written (3 x 128 B)
-# the filter kernel of each pipelined LDS tile (chebyshev_shape value); the
-# library picks 2337 at 481x321 (one round of the chip's block slots)
+# block eigensolver filter step.  In one launch of many steps (481x321: tiles
+# of 12 units); launches of RUN_STEPS steps in the counter workload
+RUN_KERNEL, RUN_STEPS = "k_cheb_run<12>", 50
+# One launch per step: the kernel of each pipelined LDS tile (chebyshev_shape
+# value; the library picks 2337 at 481x321), per row the matrix row (324 B)
+# and, for 32 vectors, x, z read and y written (3 x 128 B)
 FILTER_KERNELS = {2328: "k_cheb_ldp<2, 8>", 2337: "k_cheb_ldp<3, 7>", 2324: "k_cheb_ldp<2, 4>",
                   1328: "k_cheb_lds<2, 8, false, true>", 1337: "k_cheb_lds<3, 7, false, true>",
                   1324: "k_cheb_lds<2, 4, false, true>", 1336: "k_cheb_lds<3, 6, false, true>",
@@ -84,11 +84,11 @@ TRUTH = os.path.join(ROOT, "tests", "golden", "truth_481x321.npz")
 # the histogram stage's bytes: u16 integral images written once and read
 # once, label frames, L/a/b/texton inputs and the 96 chi-squared planes
 PMC_GROUPS = {
-    "histogram": (r"k_fill_u8|k_cue_labels|k_integral_\w+|k_band_carry|k_gradients\w*", 890.3e6),
+    "histogram": (r"k_fill_u8|k_cue_labels|k_integral_\w+|k_strip_carry|k_band_carry|k_gradients\w*", 890.3e6),
 }
 PMC_SUMMARIES = [os.path.join(ROOT, "profiles", f) for f in
-                 ("chebyshev_filter_481x321_pmc.txt", "lanczos_step_481x321_pmc.txt",
-                  "stencil_spmv_481x321_pmc.txt")]
+                 ("resident_launches_481x321_pmc.txt", "chebyshev_filter_481x321_pmc.txt",
+                  "lanczos_step_481x321_pmc.txt", "stencil_spmv_481x321_pmc.txt")]
 
 
 def parse():
@@ -104,15 +104,15 @@ def parse():
                         "for a kernel trace")
     p.add_argument("--pmc-workload", action="store_true",
                    help="run only the workload of the rocprofv3 counter passes: one 256 MiB device copy "
-                        "(calibration), 20 launches of the selected SpMV shape and 100 mixed Lanczos steps, "
-                        "then exit")
+                        "(calibration), 20 launches of the selected SpMV shape, mixed and plain Lanczos steps, "
+                        "block-solver filter steps and one k-means, then exit")
     p.add_argument("--spmv-shape", type=int, default=1, choices=sorted(SPMV_SHAPES),
                    help="SpMV launch shape for --pmc-workload (0 = k_spmv_full, else rows per lane)")
     p.add_argument("--pmc-summarize", nargs=2, metavar=("FETCH_DIR", "WRITE_DIR"),
                    help="summarise two rocprofv3 --pmc output folders (FETCH_SIZE, WRITE_SIZE passes of "
                         "--pmc-workload) into HBM bytes per launch of --kernel, calibrated on the 256 MiB copy")
     p.add_argument("--pmc-mfma", metavar="DIR",
-                   help="summarise a rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_BF16 SQ_VALU_MFMA_BUSY_CYCLES "
+                   help="summarise a rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_F32 SQ_VALU_MFMA_BUSY_CYCLES "
                         "GRBM_GUI_ACTIVE pass of --pmc-workload into MFMA FLOPs and utilisation of --kernel")
     p.add_argument("--pmc-valu", metavar="DIR",
                    help="summarise a rocprofv3 --pmc SQ_INSTS_VALU SQ_INSTS_LDS SQ_INSTS_VMEM_RD SQ_WAVES "
@@ -129,8 +129,8 @@ def parse():
 
 def pmc_mfma(d, kernel):
     """MFMA work and utilisation of `kernel` from one rocprofv3 pass with
-    SQ_INSTS_VALU_MFMA_MOPS_BF16, SQ_VALU_MFMA_BUSY_CYCLES and GRBM_GUI_ACTIVE:
-    BF16 MFMA FLOPs = 512 per MOP; utilisation = busy cycles summed over the
+    SQ_INSTS_VALU_MFMA_MOPS_F32, SQ_VALU_MFMA_BUSY_CYCLES and GRBM_GUI_ACTIVE:
+    FP32 MFMA FLOPs = 512 per MOP; utilisation = busy cycles summed over the
     SIMDs / (GPU-active cycles per XCD x 1024 SIMDs), GRBM_GUI_ACTIVE summing
     the 8 XCDs (and including the profiler's dispatch window, so the figure
     is a lower bound)."""
@@ -150,11 +150,11 @@ def pmc_mfma(d, kernel):
     if not rows:
         raise SystemExit(f"no counter rows for {kernel} under {d}")
     n = len(rows)
-    flops = sum(e["SQ_INSTS_VALU_MFMA_MOPS_BF16"] for e in rows.values()) * 512 / n
+    flops = sum(e["SQ_INSTS_VALU_MFMA_MOPS_F32"] for e in rows.values()) * 512 / n
     busy = sum(e["SQ_VALU_MFMA_BUSY_CYCLES"] for e in rows.values()) / n
     active = sum(e["GRBM_GUI_ACTIVE"] for e in rows.values()) / n
     ns = sum(e["ns"] for e in rows.values()) / n
-    print(f"{kernel} ({n} dispatches): BF16 MFMA {flops / 1e6:.1f} MFLOP per dispatch, "
+    print(f"{kernel} ({n} dispatches): FP32 MFMA {flops / 1e6:.1f} MFLOP per dispatch, "
           f"MFMA busy {busy:.0f} SIMD-cycles, GPU active {active:.0f} cycles, "
           f"MFMA utilisation >= {100 * busy / (active / 8 * 1024):.3f} %, {ns / 1e3:.1f} us under the profiler "
           f"({flops / ns / 1e3:.2f} TFLOP/s)")
@@ -285,6 +285,8 @@ def pmc_summarize(fetch_dir, write_dir, kernel):
     traffic = (f["kib"] * f["scale"] + w["kib"] * w["scale"]) * 1024
     if group:
         algo = group[1]
+    elif kernel == RUN_KERNEL:  # the matrix once, each step's block not at all: x0 read, the last block written
+        algo = (81 * 4 + 2 * 32 * 4) * W * H
     elif kernel in FILTER_KERNELS.values():
         algo = FILTER_BYTES_PER_ROW * W * H
     else:
@@ -305,9 +307,10 @@ def pmc_workload(shape):
     """Counter-pass workload: a 256 MiB copy whose FETCH_SIZE/WRITE_SIZE
     calibrate the counters (256 MiB read + 256 MiB written), then 20 stencil
     SpMVs on the 481x321 L_sym with the given launch shape, then 125 fused
-    mixed Lanczos steps (25 warm-up + 100 timed) on the same matrix, then 56
-    block-solver filter steps (default tile) on it, then one mixed-precision
-    k-means (BF16 MFMA distances) on the image's responses."""
+    mixed Lanczos steps (25 warm-up + 100 timed) on the same matrix, then 125
+    plain ones (two launches), then 56 block-solver filter steps (default tile)
+    on it, one launch each, then two launches of RUN_STEPS such steps, then one
+    k-means on the image's responses."""
     import torch
 
     import damascene_amd as dm
@@ -332,18 +335,23 @@ def pmc_workload(shape):
     ms = ctypes.c_float()
     check(lib().dmsc_lanczos_time_steps(ctx.handle, W, H, m2.data_ptr(), m2.shape[1], dm.PREC_MIXED, 100,
                                         ctypes.byref(ms)))
+    m2 = ctx.intervene(out["nmax"])
+    check(lib().dmsc_lanczos_time_steps(ctx.handle, W, H, m2.data_ptr(), m2.shape[1], dm.PREC_FP32, 100,
+                                        ctypes.byref(ms)))
     torch.cuda.synchronize()
     m3 = ctx.intervene(out["nmax"])
     ctx.convert_matrix(W, H, m3)
     with dm.tuned(resident_polls=0):  # one launch per step
         check(lib().dmsc_chebyshev_time_products(ctx.handle, W, H, m3.data_ptr(), m3.shape[1], 50, ctypes.byref(ms)))
+    check(lib().dmsc_chebyshev_time_products(ctx.handle, W, H, m3.data_ptr(), m3.shape[1], RUN_STEPS,
+                                             ctypes.byref(ms)))
     torch.cuda.synchronize()
     d_rgb = ctx.upload(dm.generate_image(W, H, CELLS, SEED))
     resp = ctx.texton_responses(ctx.rgb_to_grey(d_rgb))
     ctx.kmeans(resp, precision=dm.PREC_MIXED)
     torch.cuda.synchronize()
-    print(f"pmc workload done: copy 256 MiB, 20 x {SPMV_SHAPES[shape]}, 125 mixed Lanczos steps, "
-          "56 block-solver filter steps, one mixed k-means", flush=True)
+    print(f"pmc workload done: copy 256 MiB, 20 x {SPMV_SHAPES[shape]}, 125 mixed and 125 plain Lanczos steps, "
+          f"56 block-solver filter steps and 2 launches of {RUN_STEPS}, one k-means", flush=True)
 
 
 def step_roofline(ctx, nmax):
@@ -368,34 +376,45 @@ def step_roofline(ctx, nmax):
 
 
 def filter_roofline(ctx, nmax):
-    """Average duration of the block eigensolver's filter step (the default
-    tile, HIP events on the library's stream over FILTER_TIMED launches on
-    the image's L_sym) and its roofline: HBM on 708 algorithmic bytes per
-    row, with its FP32 multiply-adds against the FP32 peak beside it."""
+    """The block eigensolver's filter step on the image's L_sym (HIP events on
+    the library's stream over FILTER_TIMED steps): as the timed solve runs it,
+    many steps in one launch, against the FP32 matrix peak; and as one launch
+    per step, against HBM on 708 algorithmic bytes per row."""
     import damascene_amd as dm
     from damascene_amd._lib import check, lib
 
     m = ctx.intervene(nmax)
     ctx.convert_matrix(W, H, m)
     ms = ctypes.c_float()
+    args = (ctx.handle, W, H, m.data_ptr(), m.shape[1], FILTER_TIMED, ctypes.byref(ms))
     with dm.tuned(resident_polls=0):  # one launch per step
-        check(lib().dmsc_chebyshev_time_products(ctx.handle, W, H, m.data_ptr(), m.shape[1], FILTER_TIMED,
-                                                 ctypes.byref(ms)))
+        check(lib().dmsc_chebyshev_time_products(*args))
+    per_launch_s = ms.value / 1e3
+    before = ctx.resident_report()[0]
+    check(lib().dmsc_chebyshev_time_products(*args))
+    run_s = ms.value / 1e3
+    resident = ctx.resident_report()[0] > before
     tile = ctx.chebyshev_tile(W, H)
     kernel = FILTER_KERNELS.get(tile, f"filter tile {tile}")
-    avg_s = ms.value / 1e3
-    algo = FILTER_BYTES_PER_ROW * W * H
-    achieved = algo / avg_s / 1e9
-    tflops = FILTER_FLOPS_PER_ROW * W * H / avg_s / 1e12
-    return {
-        "kernel": kernel + " (block eigensolver filter step: 81-diagonal stencil product of 32 vectors, "
-                           "LDS-staged input, pipelined matrix loads)",
-        "tile": tile,
+    algo, flops = FILTER_BYTES_PER_ROW * W * H, FILTER_FLOPS_PER_ROW * W * H
+    achieved = algo / per_launch_s / 1e9
+    per_launch = {
+        "kernel": kernel + " (one launch per step, LDS-staged input, pipelined matrix loads)", "tile": tile,
         "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": pmc_traffic(kernel),
-        "avg_us": round(avg_s * 1e6, 3), "algorithmic_bytes_per_launch": algo, "launches_timed": FILTER_TIMED,
-        "valu": {"achieved_tflops": round(tflops, 2), "peak_tflops": FP32_PEAK_TFLOPS,
-                 "frac": round(tflops / FP32_PEAK_TFLOPS, 4), "flops_per_launch": FILTER_FLOPS_PER_ROW * W * H},
+        "avg_us": round(per_launch_s * 1e6, 3), "algorithmic_bytes_per_launch": algo, "launches_timed": FILTER_TIMED,
+    }
+    if not resident:
+        return {**per_launch, "step": "block eigensolver filter step"}
+    tflops = flops / run_s / 1e12
+    traffic = pmc_traffic(RUN_KERNEL)
+    return {
+        "kernel": RUN_KERNEL + " (block eigensolver filter: 81-diagonal stencil products of 32 vectors, all steps "
+                               "of an outer iteration in one launch)",
+        "bound": "fp32 mfma", "achieved": round(tflops, 2), "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
+        "frac": round(tflops / FP32_PEAK_TFLOPS, 4), "traffic": traffic and round(traffic / RUN_STEPS),
+        "avg_us": round(run_s * 1e6, 3), "flops_per_step": flops, "steps_timed": FILTER_TIMED,
+        "launch_per_step": per_launch,
     }
 
 
@@ -537,16 +556,18 @@ def stage_roofline(stage, iterations, kmeans_iterations, mixed):
     gradients (the histogram stage), [1] - [7] parabola fits, [4] eigensolve,
     [5] spectral Pb + gPb.  Each stage's algorithmic work over its window,
     against the bound it is written for: FP32 157.3 TFLOP/s (VALU and matrix
-    cores alike), HBM 8 TB/s.  The eigensolve's bytes are those of one launch
-    per step; its resident launches move fewer."""
+    cores alike), HBM 8 TB/s.  The eigensolve runs most of its steps in
+    launches that keep the matrix in registers, so it is priced by the
+    multiply-adds of its products; the parabola fits by the 11,008 non-zero
+    taps of a pixel's 96 filters."""
     n = W * H
     valu = 157.3e12
     t = [v * 1e-3 for v in stage]  # seconds
     bank = 2 * 9010 * n
     km = kmeans_iterations * 2 * n * 32 * 34
-    parabola = 2 * 58720 * n
+    parabola = 2 * 11008 * n
     hist = 890.3e6
-    eig = iterations * (FILTER_BYTES_PER_ROW if mixed else 352) * n
+    eig = iterations * 2 * 81 * (32 if mixed else 1) * n
     spb = 6272 * n
     t_bank, t_km = t[6], t[0] - t[6]
     t_hist, t_par = t[7], t[1] - t[7]
@@ -560,13 +581,13 @@ def stage_roofline(stage, iterations, kmeans_iterations, mixed):
         "histogram": {"bound": "hbm", "work": "890.3 MB (u16 integral images written once and read once, labels, "
                                               "chi-squared planes)", "ms": round(t_hist * 1e3, 3),
                       "achieved_gbs": round(hist / t_hist / 1e9, 1), "frac": round(hist / t_hist / 8e12, 4)},
-        "parabola": {"bound": "fp32 valu", "work": "2*58720 flop/px", "ms": round(t_par * 1e3, 3),
+        "parabola": {"bound": "fp32 valu", "work": "2*11008 flop/px (non-zero taps)", "ms": round(t_par * 1e3, 3),
                      "achieved_tflops": round(parabola / t_par / 1e12, 2),
                      "frac": round(parabola / t_par / valu, 4)},
-        "eigensolve": {"bound": "hbm", "ms": round(t[4] * 1e3, 3),
-                       "work": (f"{iterations} block filter products x {FILTER_BYTES_PER_ROW} B/row" if mixed else
-                                f"{iterations} Lanczos steps x 352 B/row"),
-                       "achieved_gbs": round(eig / t[4] / 1e9, 1), "frac": round(eig / t[4] / 8e12, 4)},
+        "eigensolve": {"bound": "fp32 mfma" if mixed else "exchanges between blocks", "ms": round(t[4] * 1e3, 3),
+                       "work": (f"{iterations} block products x 2*81*32 flop/px" if mixed else
+                                f"{iterations} Lanczos steps x 2*81 flop/px"),
+                       "achieved_tflops": round(eig / t[4] / 1e12, 2), "frac": round(eig / t[4] / valu, 4)},
         "spectralpb_gpb": {"bound": "fp32 mfma", "work": "6272 flop/px", "ms": round(t[5] * 1e3, 3),
                            "achieved_tflops": round(spb / t[5] / 1e12, 2), "frac": round(spb / t[5] / valu, 4)},
     }
