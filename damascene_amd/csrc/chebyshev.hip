@@ -786,10 +786,11 @@ constexpr unsigned kRunNone = ~0u;  // an entry no block has written yet
 // memory accesses.  Here every block stays resident with its pixels' matrix
 // rows in registers (81 values for each of a lane's pixels: lane 4 b + i of a
 // wave holds row i of column b of a 16 x 4 pixel unit) and a step moves only
-// the frame of its tile: 19.8 us, bound by the reads of the frames and units
-// from LDS (2.8 MB a step and block, 21,900 cycles at 128 bytes each) beside
-// 2,736 matrix instructions per SIMD (25,700 cycles at the rate a plain loop of
-// them reaches), and by the staging between them.
+// the frame of its tile: 20 us in a solve.  Of a step's 48,000 cycles the matrix
+// cores are busy for 21,900 (2,736 instructions of 8 cycles per SIMD) and LDS
+// for 14,000 (2.8 MB of frames and units per block): neither is the bound, but
+// the staging between the barriers of a half (about 8,000 cycles) overlaps with
+// nothing and the three waves of a SIMD reach the same phase together.
 //  * The 32 vectors go through LDS in two halves of 16 (a 42 x 34 frame takes
 //    91 KB); what a lane holds of the half that is not in LDS stays in
 //    registers.  A half's frame was published half a step before it is needed,
@@ -1139,7 +1140,7 @@ namespace {
 // for one launch per step.  Per product of a whole solve, with one launch per
 // step against k_cheb_run: 28.9 against 25.7 us at 481x321 (12 units), 31.0
 // against 25.3 at 512x384 (12), 26.7 against 20.2 at 400x300 (8), 21.8
-// against 20.0 at 320x240 (8).  Images that fit the device in tiles of 4 units
+// against 20.0 at 320x240 (8), 25.3 against 24.8 at 33x2100 (8).  Images that fit the device in tiles of 4 units
 // (65,536 pixels on 256 compute units) keep one launch per step: there a step
 // is one chain of dependent sums per SIMD, 14.0 against 14.7 us at 160x120.
 struct RunShape {

@@ -29,7 +29,6 @@ const int* kmeans_iterations_ptr(const void* state);  // device address of the i
 int noalloc_scratch_init(int device, void** out);
 
 // ------------------------------------------------------------- local cues
-size_t local_cues_scratch_bytes(int w, int h);
 int launch_local_cues(Ctx* ctx, int w, int h, const float* L, const float* A, const float* B, const int* tex,
                       int ntex, float* bg, float* cga, float* cgb, float* tg, int pitch, float* grads_out);
 // The local cues in two parts for two streams: part 1 the L, a, b channels

@@ -318,11 +318,12 @@ __global__ void k_lz_slots(unsigned long long* slots, int count, unsigned* z, in
 
 // `steps` plain steps from step k0 in one launch, bit-identical to
 // k_lz1<256> / k_lz2.  Two kernels per step read the 50 MB matrix (481x321)
-// for every vector and wait for two launches: 16.8 us a step.  Here every
+// for every vector and wait for two launches: 13.5 us a step (16.5 with the
+// 2,048-row blocks k_lz2 had before).  Here every
 // block stays resident, so each lane keeps its row's 81 matrix entries, its z
 // and its last q in registers and a step moves the stencil halo of z, the
 // basis row and two partial sums per block: 5.9 us, bound by the two
-// exchanges (about 3,800 cycles each of 15,000) and the 81 LDS reads per row
+// exchanges (about 3,800 cycles each of 14,200) and the 81 LDS reads per row
 // (3,500).
 //  * Rows are consecutive, so halo and sums keep the linear indexing and the
 //    order of the two-kernel step.

@@ -887,16 +887,6 @@ void release_local_cues(const Ctx* ctx) {
   plan_caches().erase(ctx);
 }
 
-size_t local_cues_scratch_bytes(int w, int h) {
-  const int bw = w + 2 * kBorder, bh = h + 2 * kBorder;
-  // generous bound: rotated frames are at most (bw+bh)^2
-  const size_t rot = (size_t)(bw + bh) * (bw + bh);
-  const size_t lab = 16 * (rot + 256);
-  const size_t ints = (12 * 32 + 4 * 64) * rot * sizeof(uint16_t);  // texture frames at up to 64 bins
-  const size_t grads = (size_t)4 * 24 * w * h * sizeof(float);
-  return lab + ints + grads + 4096;
-}
-
 // localcues.cu:257-300 localCues, in two parts that may run on two streams:
 // part 1 the L, a and b channels (frames 0..11: labels, integral images,
 // Bg and Cg gradients and their parabola fits), which do not need the

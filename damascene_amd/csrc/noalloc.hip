@@ -26,8 +26,9 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
 
-// The largest input: what the array held when |x|^2 was kept per pixel, and
-// the documented limit.  The k-means state alone is needed now.
+// The largest input, documented and reported by dmsc_kmeans_noalloc_max_pixels:
+// what the array holds with |x|^2 kept per pixel.  The k-means state alone is
+// needed now; the limit stays, so that what was refused stays refused.
 constexpr long kMaxPixels = 2092608;
 
 }  // namespace
