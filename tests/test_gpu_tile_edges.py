@@ -1,5 +1,7 @@
 """Kernels at the sizes where their tiles, chunks and dispatch rules end,
 against the CPU oracle (bit for bit) or an FP64 reference."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -318,3 +320,18 @@ def test_affinity_padding(ctx, w, h, pad):
         print(f"{tight:.0f} us at pitch {ref.shape[1]}, {wide:.0f} us at {pitch}", flush=True)
         # twice the bytes written; ten times leaves room for any launch effect
         assert wide < 10 * tight
+
+
+# both precisions take exact distances: the same labels, nothing recomputed
+@pytest.mark.parametrize("k", [32, 64])
+def test_kmeans_recomputes_nothing(ctx, k):
+    print(f"case: k-means re-checks, {k} clusters", flush=True)
+    resp = ctx.upload((np.random.RandomState(k).randn(34, 61, 83) * 0.1).astype(np.float32))
+    out = []
+    for precision in (dm.PREC_FP32, dm.PREC_MIXED):
+        labels, it = ctx.kmeans(resp, k=k, precision=precision)
+        n = ctypes.c_int(-1)
+        check(lib().dmsc_kmeans_rechecks(ctx.handle, ctypes.byref(n)))
+        assert n.value == 0
+        out.append((host(labels).tobytes(), it))
+    assert out[0] == out[1]
